@@ -118,6 +118,9 @@ def chunk_launches(steps, chunk, window):
     return sum(-(-k // window) for k in sizes)
 
 
+RESIDENT_STEPS = 16384  # steps of one resident launch at most (hs_runtime.hip)
+
+
 def run_form(spec, prec, engine, steps, settle, options=None):
     """Build, settle `settle` untimed steps (the network leaves its quiescent
     start), instantiate every graph the timed run launches (hs_net_prepare), then
@@ -149,6 +152,7 @@ def run_form(spec, prec, engine, steps, settle, options=None):
         "window": window,
         "window_launches": chunk_launches(steps, net.get_option(rt.OPT_GRAPH_CHUNK), window),
         "build_s": build_s,
+        "resident": net.get_option(rt.OPT_WAS_RESIDENT) == 1,
     }
     res["events_per_s"] = res["events"] / res["wall_s"]
     res["sim_s_per_wall_s"] = steps * spec.dt / res["wall_s"]
@@ -742,7 +746,18 @@ def main():
             }[name]
 
         name = max(kt, key=lambda k: kt[k]["total_ms"])
-        if len(kt) == 1 and name == "hs_k_window":
+        if fp32["resident"]:
+            # the timed form's only kernel (the kernel-timed run, an event pair per
+            # launch, takes the per-step kernels instead): the same bytes a step,
+            # over the timed run's own time
+            name = "hs_k_resident"
+            launches = -(-steps // RESIDENT_STEPS)
+            steps_per_launch = steps / launches
+            bpl = per_step("hs_k_window", fp32["spikes_per_step"], fp32["events_per_step"]) * steps_per_launch
+            avg_us = fp32["gpu_ms"] * 1e3 / launches
+            src = "timed run: its HIP events over its resident launches; bytes from its own spike and event counts"
+            ev_launch = fp32["events_per_step"] * steps_per_launch
+        elif len(kt) == 1 and name == "hs_k_window":
             # the dominant kernel is the timed form's only kernel: its bytes and
             # its launch time both from the timed run itself (HIP events around
             # its steps on the runtime's stream, over its launches)
@@ -765,8 +780,10 @@ def main():
                     "frac": round(achieved / HBM_PEAK_GBS, 6), "traffic": measured_traffic(args, name),
                     "kernel": name, "bytes_per_launch": int(bpl), "steps_per_launch": round(steps_per_launch, 3),
                     "avg_launch_us": round(avg_us, 3), "avg_launch_from": src,
-                    "avg_launch_us_event_pairs": round(kt[name]["avg_us"], 3),
+                    "avg_launch_us_event_pairs": round(kt[name]["avg_us"], 3) if name in kt else None,
                     "kernels": {k: {kk: round(vv, 3) for kk, vv in v.items()} for k, v in kt.items()}}
+        if fp32["resident"]:  # (its effects are LDS atomics: the comparison is per window of the per-step forms)
+            ev_launch, avg_us = fp32["events_per_step"] * W, fp32["gpu_ms"] * 1e3 / steps * W
         roofline["atomics"] = atomic_ceiling(N, ev_launch, avg_us, args.seed)
         log("atomics", roofline["atomics"])
 

@@ -10,8 +10,6 @@
 #include "hs_model_exprs.h"
 #include "hs_philox.h"
 
-#define HS_WAVE 64
-
 __device__ __forceinline__ int hs_lane() { return threadIdx.x & (HS_WAVE - 1); }
 
 /*
@@ -159,14 +157,14 @@ template <typename R, int C> struct HsCg;
 template <int MODEL> struct HsNV {
     static constexpr int value = HsCg<double, MODEL - HS_MODEL_CODE>::NV;
 };
-template <int MODEL> __device__ constexpr bool hs_cg_noisy()
+template <int MODEL> __host__ __device__ constexpr bool hs_cg_noisy()
 {
     if constexpr (HS_IS_CODE_MODEL(MODEL)) return HsCg<double, MODEL - HS_MODEL_CODE>::NOISY != 0;
     else return false;
 }
 #else
 template <int MODEL> struct HsNV;
-template <int MODEL> __device__ constexpr bool hs_cg_noisy() { return false; }
+template <int MODEL> __host__ __device__ constexpr bool hs_cg_noisy() { return false; }
 #endif
 template <> struct HsNV<HS_MODEL_LIF_CUBA> { static constexpr int value = HS_LIF_CUBA_NVARS; };
 template <> struct HsNV<HS_MODEL_LIF_NOISE> { static constexpr int value = HS_LIF_NOISE_NVARS; };
@@ -217,6 +215,80 @@ __device__ __forceinline__ bool hs_neuron_step(R *s, const R *k, int not_ref, R 
         HsOps<R>::hh(s, k);
     }
     return (s[0] > vth) && not_ref;
+}
+
+/* what a step reads of its group's descriptor besides the constants k[]: a loop
+   over many steps reads it once */
+template <typename R>
+struct HsStepK {
+    R vth, vr;
+    double dt;
+    unsigned long long seed;
+    unsigned int stream;
+    int has_reset, ref_steps, nst;
+    __device__ __forceinline__ explicit HsStepK(const DGroup<R> &g)
+        : vth(g.vth), vr(g.vr), dt(g.dt), seed(g.seed), stream(g.stream), has_reset(g.has_reset),
+          ref_steps(g.ref_steps), nst(g.nst)
+    {
+    }
+};
+
+/* one step of one neuron: deferred reset, StateMonitor samples, update, threshold; returns the spike */
+template <typename R, int MODEL, bool FUSED>
+__device__ __forceinline__ bool hs_step_one(const DGroup<R> &g, const HsStepK<R> &c, R *s, const R *k, int32_t &last,
+                                            long long t, int i, long long no_reset_before, R xi)
+{
+    constexpr int NV = HsNV<MODEL>::value;
+    if constexpr (MODEL == HS_MODEL_SPIKEGEN) { /* spikegenerator.cu:43-80: no state, no refractoriness */
+        const bool fire = hs_spikegen_fires(g, t, i);
+        if (fire) last = (int32_t)t;
+        return fire;
+    } else if constexpr (MODEL == HS_MODEL_POISSON) { /* PoissonGroup: rand() < rates*dt */
+        const R p = s[0] * k[0];
+        const bool fire = hs_rand(c.seed, c.stream, (uint32_t)i, t) < (double)p;
+        if (fire) last = (int32_t)t;
+        return fire;
+    } else {
+        if (c.has_reset && (long long)last == t - 1 && t - 1 >= no_reset_before) {
+#ifdef HS_CG_MODELS
+            if constexpr (HS_IS_CODE_MODEL(MODEL))
+                HsCg<R, MODEL - HS_MODEL_CODE>::reset(s, (R)c.dt, (double)(t - 1) * c.dt, i, c.seed, c.stream,
+                                                      t - 1);
+            else
+#endif
+                s[0] = c.vr;
+        }
+        for (int m = 0; m < c.nst; ++m) {
+            /* the row of step t (uniform over the launch), then this neuron's column */
+            const long long dt0 = t - g.st_t0[m];
+            if (dt0 < 0) continue;
+            const int every = g.st_every[m];
+            const long long row = every == 1 ? dt0 : dt0 / every;
+            if (row * every != dt0 || row >= g.st_rows[m]) continue;
+            int col;
+            if (g.st_map[m]) col = hs_ld(g.st_map[m] + i);
+            else col = (i >= g.st_start[m] && i < g.st_stop[m]) ? i - g.st_start[m] : -1;
+            if (col >= 0) {
+                const int sv = g.st_var[m];
+                R val = hs_opaque(s[0]);
+#pragma unroll
+                for (int v = 1; v < NV; ++v) val = sv == v ? hs_opaque(s[v]) : val;
+                hs_st(g.st_buf[m] + row * (long long)g.st_width[m] + col, val);
+            }
+        }
+        const int not_ref = (t - (long long)last) >= (long long)c.ref_steps;
+        bool spk;
+#ifdef HS_CG_MODELS
+        if constexpr (HS_IS_CODE_MODEL(MODEL))
+            spk = HsCg<R, MODEL - HS_MODEL_CODE>::step(s, not_ref, xi, (R)c.dt, (double)t * c.dt, i, c.seed, c.stream,
+                                                       t) &&
+                  not_ref;
+        else
+#endif
+            spk = hs_neuron_step<R, MODEL>(s, k, not_ref, c.vth, xi);
+        if (spk) last = (int32_t)t;
+        return spk;
+    }
 }
 
 /* ------------------------------------------------------------------------ */

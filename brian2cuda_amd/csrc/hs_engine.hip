@@ -173,64 +173,6 @@ __device__ __forceinline__ void hs_push_near(const HsPush<R> &ps, int gid, int i
     if (hs_lane() == 0 && emitted) hs_atomic_add(ps.emit, emitted);
 }
 
-/* one step of one neuron inside the update window; returns the spike */
-template <typename R, int MODEL, bool FUSED>
-__device__ __forceinline__ bool hs_step_one(const DGroup<R> &g, R *s, const R *k, int32_t &last, long long t, int i,
-                                            long long no_reset_before, R xi)
-{
-    constexpr int NV = HsNV<MODEL>::value;
-    if constexpr (MODEL == HS_MODEL_SPIKEGEN) { /* spikegenerator.cu:43-80: no state, no refractoriness */
-        const bool fire = hs_spikegen_fires(g, t, i);
-        if (fire) last = (int32_t)t;
-        return fire;
-    } else if constexpr (MODEL == HS_MODEL_POISSON) { /* PoissonGroup: rand() < rates*dt */
-        const R p = s[0] * k[0];
-        const bool fire = hs_rand(g.seed, g.stream, (uint32_t)i, t) < (double)p;
-        if (fire) last = (int32_t)t;
-        return fire;
-    } else {
-        if (g.has_reset && (long long)last == t - 1 && t - 1 >= no_reset_before) {
-#ifdef HS_CG_MODELS
-            if constexpr (HS_IS_CODE_MODEL(MODEL))
-                HsCg<R, MODEL - HS_MODEL_CODE>::reset(s, (R)g.dt, (double)(t - 1) * g.dt, i, g.seed, g.stream,
-                                                      t - 1);
-            else
-#endif
-                s[0] = g.vr;
-        }
-        for (int m = 0; m < g.nst; ++m) {
-            /* the row of step t (uniform over the launch), then this neuron's column */
-            const long long dt0 = t - g.st_t0[m];
-            if (dt0 < 0) continue;
-            const int every = g.st_every[m];
-            const long long row = every == 1 ? dt0 : dt0 / every;
-            if (row * every != dt0 || row >= g.st_rows[m]) continue;
-            int col;
-            if (g.st_map[m]) col = hs_ld(g.st_map[m] + i);
-            else col = (i >= g.st_start[m] && i < g.st_stop[m]) ? i - g.st_start[m] : -1;
-            if (col >= 0) {
-                const int sv = g.st_var[m];
-                R val = hs_opaque(s[0]);
-#pragma unroll
-                for (int v = 1; v < NV; ++v) val = sv == v ? hs_opaque(s[v]) : val;
-                hs_st(g.st_buf[m] + row * (long long)g.st_width[m] + col, val);
-            }
-        }
-        const int not_ref = (t - (long long)last) >= (long long)g.ref_steps;
-        bool spk;
-#ifdef HS_CG_MODELS
-        if constexpr (HS_IS_CODE_MODEL(MODEL))
-            spk = HsCg<R, MODEL - HS_MODEL_CODE>::step(s, not_ref, xi, (R)g.dt, (double)t * g.dt, i, g.seed, g.stream,
-                                                       t) &&
-                  not_ref;
-        else
-#endif
-            spk = hs_neuron_step<R, MODEL>(s, k, not_ref, g.vth, xi);
-        if (spk) last = (int32_t)t;
-        return spk;
-    }
-}
-
 template <typename R, int MODEL, bool FUSED, bool PUSH>
 __device__ __forceinline__ void hs_update_tile(const DGroup<R> &g, int gid, int tile, long long T, int w, int wmax,
                                                long long no_reset_before, HsCompactLdsW *L,
@@ -321,7 +263,8 @@ __device__ __forceinline__ void hs_update_tile(const DGroup<R> &g, int gid, int 
 #pragma unroll
                 for (int m = 0; m + 1 < (NOISY ? HS_MAX_WINDOW : 1); ++m) xi[m] = xi[m + 1];
             }
-            if (hs_step_one<R, MODEL, FUSED>(g, s, k, last, T + j, i, no_reset_before, xj)) bits |= 1u << j;
+            if (hs_step_one<R, MODEL, FUSED>(g, HsStepK<R>(g), s, k, last, T + j, i, no_reset_before, xj))
+                bits |= 1u << j;
         }
     }
     if (valid) {

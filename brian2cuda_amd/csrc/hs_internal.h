@@ -37,6 +37,9 @@ typedef unsigned long long uint64_t;
 #define HS_MAX_DELAY_SLOTS 4096 /* D per pathway (LDS prefix table) */
 #define HS_MAX_WINDOW 8         /* steps per update launch of the windowed form */
 #define HS_GTILE 256            /* targets per block of the gather delivery */
+#define HS_WAVE 64
+#define HS_RES_MAXT 512         /* resident loop: neurons (threads) of a block at most */
+#define HS_RES_HELPERS 256      /* and its threads that only deliver (models with noise): one per line */
 
 /* delivery modes of a pathway */
 #define HS_DELIVER_SCATTER 1 /* per (pre, delay) bundles, global atomics on the targets */
@@ -58,7 +61,8 @@ struct HsCtl {
     long long no_reset_before; /* resets of spikes at steps < this were already applied */
     unsigned long long pending; /* pipelined windows: events of emitted spikes still in flight at base */
     unsigned long long scatter_bad; /* hs_scatter_add: indices outside the target array */
-    unsigned long long pad_[12];
+    unsigned long long stalled; /* resident loop: a block waited in vain for the others' spikes */
+    unsigned long long pad_[11];
     unsigned long long ev_slot[HS_EV_SLOTS * HS_EV_STRIDE];  /* synaptic events delivered: sum of ev_slot[k*STRIDE] */
     unsigned long long spk_slot[HS_EV_SLOTS * HS_EV_STRIDE]; /* spikes emitted, spread the same way */
 };
@@ -177,6 +181,42 @@ struct DPath {
     int npr;
     int post_read_var[HS_MAX_VARS];
     const int32_t *synpre;
+};
+
+/*
+ * The resident step loop (hs_resident.h): the synapses laid out by (source,
+ * owning block), the blocks' mail and the geometry; it lies in HBM
+ * beside the group descriptors.
+ */
+/* one synapse of a (source, owning block) segment: its target's index in the
+   block | target variable's plane << 10 | delay << 16, and its weight */
+template <typename R> struct HsResSyn;
+template <> struct __attribute__((aligned(8))) HsResSyn<float> {
+    uint32_t pack;
+    float w;
+};
+template <> struct __attribute__((aligned(16))) HsResSyn<double> {
+    double w;
+    uint32_t pack, pad;
+};
+
+template <typename R>
+struct HsResArgs {
+    const int32_t *off;      /* segment of (pre, block b): syn[off[pre*nb + b] .. off[pre*nb + b + 1]) */
+    const HsResSyn<R> *syn;
+    unsigned long long *mail; /* [depth][nb][mwords]: a line per block and window (hs_res_header) */
+    unsigned long long *bits; /* [nhist][nb][waves]: spikes of step t as ballots in row t mod nhist */
+    HsCtl *ctl;
+    int n, nb, nown, W, dmax, nslots, nhist, depth, mwords, hwords, lanes_log2, list_cap, cap;
+    int nplanes;
+    int plane[HS_MAX_VARS];  /* accumulator plane of variable v, or -1 */
+    int o_acc, o_evw, o_list, o_list2, o_cnt, o_big, o_evt, o_stage, lds; /* LDS offsets (hs_res_offsets), total */
+};
+
+/* a resident run's totals, in host memory */
+struct HsResInfo {
+    long long base;
+    unsigned long long events, spikes, records, stalled;
 };
 
 /*
@@ -330,6 +370,27 @@ hipError_t hs_launch_window(const DGroup<R> *groups, int ng, int total_tiles, co
 template <typename R>
 hipError_t hs_launch_pending(const DPath<R> *paths, int np, HsCtl *ctl, hipStream_t s);
 hipError_t hs_launch_tick(HsCtl *ctl, long long k, hipStream_t s);
+/* resident step loop (hs_resident.hip).  offsets: the LDS layout; layout: entries
+   per (source, block) segment into cnt (and the segments that have any into
+   *nonempty), or (write) the entries themselves;
+   resident: nsteps steps from T0, windows numbered from win0 (ms as above: one
+   group of a built-in model with synapses); close: spike lists, step base and
+   totals after it; refill: the accumulators of the pipelined windows, for a
+   network that goes back to them.  a is the host's copy, da the one in HBM */
+template <typename R>
+void hs_res_offsets(HsResArgs<R> *a, int plain);
+int hs_res_hwords(int ms); /* header words of a line */
+template <typename R>
+hipError_t hs_launch_res_layout(const DPath<R> *paths, int np, const HsResArgs<R> &a, int32_t *cnt,
+                                unsigned long long *nonempty, bool write, hipStream_t s);
+template <typename R>
+hipError_t hs_launch_resident(const HsResArgs<R> &a, const HsResArgs<R> *da, const DGroup<R> *g, int ms, int plain,
+                              int block, long long T0, int nsteps, uint32_t win0, hipStream_t s);
+template <typename R>
+hipError_t hs_launch_res_close(const HsResArgs<R> &a, const DGroup<R> *g, int block, long long T0, int nsteps,
+                               HsResInfo *info, hipStream_t s);
+template <typename R>
+hipError_t hs_launch_res_refill(const DPath<R> *paths, int np, HsCtl *ctl, int W, hipStream_t s);
 /* resets of spikes before ctl->base are applied (after a finalize) */
 hipError_t hs_launch_mark_reset(HsCtl *ctl, hipStream_t s);
 /* STDP pathways at step ctl->base + koff (plain form, after the delivery of the

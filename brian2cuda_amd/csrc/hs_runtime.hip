@@ -493,6 +493,25 @@ static int64_t hs_mon_rows(const HMon &M, int64_t step)
     return (step - M.t0 + M.every - 1) / M.every;
 }
 
+/* a network's resident step loop: what hs_k_resident is launched with */
+struct HsResNet {
+    int state = 0;       /* 0 not decided yet, 1 laid out, -1 not for this network */
+    bool active = false; /* the last run was resident */
+    int64_t asked = 0;   /* steps run in the per-step forms so far */
+    int block = 0;
+    uint32_t win = 1;    /* number of the next window */
+    size_t mail_bytes = 0;
+    HsResInfo *info = nullptr; /* pinned */
+    uint64_t ev_bias = 0;      /* events the pipelined windows counted at emission, delivered (and counted) again here */
+    HsResArgs<double> a64 = {}; /* geometry and pointers, by precision; and their copy in HBM */
+    HsResArgs<float> a32 = {};
+    void *dargs = nullptr;
+};
+
+template <typename R> static HsResArgs<R> &hs_res_args(HsResNet &r);
+template <> HsResArgs<double> &hs_res_args<double>(HsResNet &r) { return r.a64; }
+template <> HsResArgs<float> &hs_res_args<float>(HsResNet &r) { return r.a32; }
+
 struct hs_net {
     int prec, engine;
     double dt;
@@ -512,8 +531,8 @@ struct hs_net {
     int64_t step = 0;
     /* 0 update block, 1 scatter grid, 2 graph chunk, 3 fused delivery blocks,
        4 window, 5 delivery mode, 6 gather block, 7 kernel timing, 8 noise blocks,
-       9 pipelined windows */
-    long long opt[12] = {256, 0, 256, 0, 0, 0, 256, 0, 0, 0, 0, 0};
+       9 pipelined windows, 10 update grid, 11 fast math, 12 resident step loop */
+    long long opt[13] = {256, 0, 256, 0, 0, 0, 256, 0, 0, 0, 0, 0, 1};
     /* kernel timing: event pairs of the current run, totals per kind */
     std::vector<hipEvent_t> kt_pool;
     std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> kt_open;
@@ -530,6 +549,7 @@ struct hs_net {
     std::vector<HsCgModel> cg_models;  /* code models, ids HS_MODEL_CODE + index */
     std::vector<HsSynCgModel> cg_syn;  /* synaptic code of the pathways with HS_DELIVER_CODE */
     const HsCgKernels *cg = nullptr;   /* their compiled kernels (from the first run) */
+    HsResNet res;                      /* the resident step loop */
 };
 
 static size_t hs_rsize(const hs_net *net) { return net->prec == HS_F64 ? sizeof(double) : sizeof(float); }
@@ -596,6 +616,7 @@ extern "C" void hs_net_destroy(hs_net *net)
     (void)hipStreamSynchronize(g_rt.stream);
     hs_drop_graphs(net);
     for (void *p : net->allocs) (void)hipFree(p);
+    if (net->res.info) (void)hipHostFree(net->res.info);
     if (net->ev0) (void)hipEventDestroy(net->ev0);
     if (net->ev1) (void)hipEventDestroy(net->ev1);
     for (auto &o : net->kt_open) {
@@ -1736,7 +1757,8 @@ extern "C" int hs_net_get_rate_monitor(hs_net *net, int mid, double *rate, int64
 
 extern "C" int hs_net_set_option(hs_net *net, int key, long long value)
 {
-    if (!net || key < 0 || key > 11) return hs_fail(HS_ERR_ARG, "bad option key");
+    if (!net || key < 0 || key > 12) return hs_fail(HS_ERR_ARG, "bad option key");
+    if (key == 12 && (value < 0 || value > 1)) return hs_fail(HS_ERR_ARG, "resident step loop: 0 off, 1 on");
     if (key == 7 && (value < 0 || value > 1)) return hs_fail(HS_ERR_ARG, "kernel timing: 0 off, 1 on");
     if (key == 11 && (value < 0 || value > 1)) return hs_fail(HS_ERR_ARG, "fast math: 0 off, 1 on");
     if (key == 11 && value && net->prec != HS_F32)
@@ -1767,8 +1789,8 @@ extern "C" int hs_net_set_option(hs_net *net, int key, long long value)
 
 extern "C" int hs_net_get_option(hs_net *net, int key, long long *value)
 {
-    if (!net || key < 0 || key > 11 || !value) return hs_fail(HS_ERR_ARG, "bad option key");
-    *value = net->opt[key];
+    if (!net || key < 0 || key > 13 || !value) return hs_fail(HS_ERR_ARG, "bad option key");
+    *value = key == 13 ? (net->res.active ? 1 : 0) : net->opt[key];
     return HS_OK;
 }
 
@@ -2318,13 +2340,17 @@ static int hs_prepare_run(hs_net *net, int64_t nsteps)
     return HS_OK;
 }
 
+static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use);
+
 extern "C" int hs_net_prepare(hs_net *net, int64_t nsteps)
 {
     if (!net) return hs_fail(HS_ERR_ARG, "null net");
     if (nsteps < 0) return hs_fail(HS_ERR_ARG, "negative step count");
     if (net->g.empty()) return hs_fail(HS_ERR_STATE, "network has no groups");
     HS_TRY(hs_prepare_run(net, nsteps));
-    if (net->opt[2] <= 0 || net->opt[7] || nsteps == 0) return HS_OK;
+    bool resident = false;
+    HS_TRY(hs_res_ready(net, nsteps, &resident));
+    if (resident || net->opt[2] <= 0 || net->opt[7] || nsteps == 0) return HS_OK;
     const int64_t K = net->opt[2];
     hipGraphExec_t exec;
     if (nsteps >= K) HS_TRY(hs_chunk_graph(net, K, &exec));
@@ -2368,12 +2394,327 @@ static int hs_check_spike_monitors(hs_net *net, int64_t k, bool *resized)
     return HS_OK;
 }
 
+/* ------------------------------------------------------------------------ */
+/* the resident step loop (hs_resident.h)                                    */
+/* ------------------------------------------------------------------------ */
+
+#define HS_RES_MIN_STEPS 10
+#define HS_RES_SYN_PER_STEP 50000
+
+/* LDS a block may use: the compute unit's 160 KiB, with a margin */
+#define HS_RES_LDS (156 * 1024)
+
+/* geometry of the resident loop, or false: more than one group, a model the
+   loop is not compiled for, pathways of other kinds, more neurons than the
+   chip's blocks own, delays or sums that do not fit LDS */
+template <typename R>
+static bool hs_res_geometry(hs_net *net)
+{
+    HsResNet &r = net->res;
+    HsResArgs<R> &a = hs_res_args<R>(r);
+    if (net->g.size() != 1 || net->p.empty() || net->n_gather || net->n_plastic || !net->cg_syn.empty() ||
+        !net->cg_models.empty())
+        return false;
+    const HGroup &g = net->g[0];
+    if (g.model != HS_MODEL_LIF_CUBA && g.model != HS_MODEL_LIF_NOISE && g.model != HS_MODEL_HH_COBA) return false;
+    for (const HMon &M : net->m)
+        if (M.kind == 3) return false;
+    int64_t total = 0;
+    int dmin = 1 << 30, dmax = 0;
+    for (int v = 0; v < HS_MAX_VARS; ++v) a.plane[v] = -1;
+    a.nplanes = 0;
+    for (const HPath &P : net->p) {
+        if (P.dmode != HS_DELIVER_SCATTER) return false;
+        total += P.nsyn;
+        dmin = std::min(dmin, P.dmin);
+        dmax = std::max(dmax, P.dmax);
+        if (a.plane[P.var] < 0) a.plane[P.var] = a.nplanes++;
+    }
+    if (total >= 0x7fffffffLL || dmax > 1000) return false;
+    /* blocks of whole waves, at least as many threads as there are blocks (each
+       thread then reads one line) and at most one block per compute unit: up to
+       four waves a block have a SIMD each, and fewer lines cost less */
+    a.ctl = net->ctl;
+    a.n = g.n;
+    const int most = std::min(g_rt.n_cu, 256);
+    r.block = HS_WAVE;
+    while (r.block <= HS_RES_MAXT && (g.n + r.block - 1) / r.block > std::min(most, r.block)) r.block += HS_WAVE;
+    a.nb = std::min(most, (g.n + r.block - 1) / r.block);
+    if (r.block > 256) a.nb = most; /* more than a wave per SIMD: every compute unit */
+    a.nown = (g.n + a.nb - 1) / a.nb;
+    r.block = (a.nown + HS_WAVE - 1) / HS_WAVE * HS_WAVE;
+    if (r.block > HS_RES_MAXT) return false;
+    a.dmax = dmax;
+    a.nslots = dmax + 1;
+    a.nhist = std::max(1, dmax);
+    a.W = std::min(HS_MAX_WINDOW, dmin + 1);
+    a.hwords = hs_res_hwords(g.model);
+    a.mwords = ((a.hwords + (a.nown * a.W + 1) / 2) + 15) / 16 * 16;
+    a.list_cap = std::max(256, 4 * a.hwords * a.nb);
+    a.lanes_log2 = 0; /* with the layout */
+    a.cap = 0;
+    const int plain = net->engine == HS_ENGINE_PLAIN;
+    /* the windows whose lines are read: the current one, and in the plain form
+       those that an overflowing bucket reads back */
+    a.depth = plain ? (dmax + a.W - 1) / a.W + 3 : 2;
+    hs_res_offsets<R>(&a, plain);
+    if (a.lds > HS_RES_LDS) return false;
+    if (plain) {
+        const size_t rest = (size_t)a.lds + 64;
+        a.cap = (int)std::min<size_t>(2048, (HS_RES_LDS - rest) / ((size_t)a.nslots * (sizeof(R) + sizeof(uint16_t))));
+        if (a.cap < 16) return false;
+        hs_res_offsets<R>(&a, plain);
+    }
+    return true;
+}
+
+/* lays the network's synapses out for the resident loop and allocates its mail;
+   the network stays in the per-step forms (state -1) when memory runs out */
+template <typename R>
+static int hs_res_layout(hs_net *net)
+{
+    HsResNet &r = net->res;
+    HsResArgs<R> &a = hs_res_args<R>(r);
+    const int np = (int)net->p.size();
+    int64_t total = 0;
+    for (const HPath &P : net->p) total += P.nsyn;
+    const long long segs = (long long)a.n * a.nb;
+    const int nblk = hs_scan_blocks(segs);
+    int32_t *cnt = nullptr;
+    long long *bsum = nullptr;
+    r.mail_bytes = sizeof(unsigned long long) * (size_t)a.depth * a.nb * a.mwords;
+    const size_t bits_bytes = sizeof(unsigned long long) * (size_t)a.nhist * a.nb * (r.block / HS_WAVE);
+    bool ok = hipMalloc((void **)&cnt, sizeof(int32_t) * (size_t)segs) == hipSuccess &&
+              hipMalloc((void **)&bsum, sizeof(long long) * (size_t)(nblk + 1)) == hipSuccess &&
+              hipHostMalloc((void **)&r.info, sizeof(HsResInfo), hipHostMallocDefault) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    void *syn = nullptr, *off = nullptr;
+    ok = ok && hs_dalloc(net, sizeof(int32_t) * (size_t)(segs + 1), &off, false) == HS_OK &&
+         hs_dalloc(net, sizeof(HsResSyn<R>) * (size_t)std::max<int64_t>(total, 1), &syn, false) == HS_OK &&
+         hs_dalloc(net, r.mail_bytes, (void **)&a.mail, true) == HS_OK &&
+         hs_dalloc(net, bits_bytes, (void **)&a.bits, false) == HS_OK &&
+         hs_dalloc(net, sizeof(HsResArgs<R>), &r.dargs, false) == HS_OK;
+    a.off = (const int32_t *)off;
+    a.syn = (const HsResSyn<R> *)syn;
+    hipError_t e = hipSuccess;
+    if (ok) {
+        memset(r.info, 0, sizeof(HsResInfo));
+        const DPath<R> *dp = (const DPath<R> *)net->dpaths;
+        unsigned long long *nonempty = &net->ctl->pending, some = 0; /* (a word that each use writes anew) */
+        e = hipMemsetAsync(nonempty, 0, sizeof(some), g_rt.stream);
+        if (e == hipSuccess) e = hs_launch_res_layout<R>(dp, np, a, cnt, nonempty, false, g_rt.stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(&some, nonempty, sizeof(some), hipMemcpyDeviceToHost, g_rt.stream);
+        if (e == hipSuccess) e = hs_launch_scan(cnt, segs, bsum, (int32_t *)off, g_rt.stream);
+        if (e == hipSuccess) e = hs_launch_res_layout<R>(dp, np, a, cnt, nonempty, true, g_rt.stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(g_rt.stream);
+        /* threads per spike: a thread keeps four entries in flight, and most
+           segments (half as long again as the mean of those that are not empty)
+           should take one round */
+        const double seg = (double)total / (double)std::max(1ull, some);
+        while (a.lanes_log2 < 6 && 1.5 * seg > 4.0 * (1 << a.lanes_log2)) a.lanes_log2++;
+        if (e == hipSuccess) e = hipMemcpyAsync(r.dargs, &a, sizeof(a), hipMemcpyHostToDevice, g_rt.stream);
+    }
+    const hipError_t es = hipStreamSynchronize(g_rt.stream);
+    if (cnt) (void)hipFree(cnt);
+    if (bsum) (void)hipFree(bsum);
+    if (!ok) {
+        void *held[] = {off, syn, a.mail, a.bits, r.dargs};
+        for (void *p : held) hs_dfree(net, p);
+        if (r.info) (void)hipHostFree(r.info);
+        r.dargs = nullptr;
+        r.info = nullptr;
+        r.state = -1;
+        return HS_OK;
+    }
+    HS_HIP(e);
+    HS_HIP(es);
+    r.state = 1;
+    return HS_OK;
+}
+
+/* whether this run of nsteps steps is resident; lays the synapses out on the
+   first one that is */
+template <typename R>
+static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use)
+{
+    HsResNet &r = net->res;
+    *use = false;
+    if (r.state < 0 || !net->opt[12] || net->opt[7] || nsteps == 0) return HS_OK;
+    if (r.state == 0) {
+        if (!hs_res_geometry<R>(net)) {
+            r.state = -1;
+            return HS_OK;
+        }
+        /* the layout is worth its time once the steps asked for gain as much: 30 ps a
+           synapse (with the allocations) against 1.5 us a step at least, so a
+           network that runs a few steps over many synapses stays in the per-step
+           forms, and one that goes on changes over */
+        int64_t total = 0;
+        for (const HPath &P : net->p) total += P.nsyn;
+        if (r.asked + nsteps < HS_RES_MIN_STEPS + total / HS_RES_SYN_PER_STEP) return HS_OK;
+        HS_TRY(hs_res_layout<R>(net));
+        if (r.state < 0) return HS_OK;
+    }
+    *use = true;
+    return HS_OK;
+}
+
+static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use)
+{
+    return net->prec == HS_F64 ? hs_res_ready<double>(net, nsteps, use) : hs_res_ready<float>(net, nsteps, use);
+}
+
+/* events still in flight at the network's step (ctl->pending) */
+static int hs_pending(hs_net *net, uint64_t *out)
+{
+    if (net->prec == HS_F64)
+        HS_HIP(hs_launch_pending<double>((const DPath<double> *)net->dpaths, (int)net->p.size(), net->ctl, g_rt.stream));
+    else
+        HS_HIP(hs_launch_pending<float>((const DPath<float> *)net->dpaths, (int)net->p.size(), net->ctl, g_rt.stream));
+    unsigned long long p = 0;
+    HS_HIP(hipMemcpyAsync(&p, &net->ctl->pending, sizeof(p), hipMemcpyDeviceToHost, g_rt.stream));
+    HS_HIP(hipStreamSynchronize(g_rt.stream));
+    *out = p;
+    return HS_OK;
+}
+
+/* from the per-step forms to the resident loop: the state is complete between
+   runs and the spikes in flight are in the lists; only the event count differs
+   (the pipelined windows count at emission, the loop at arrival) */
+static int hs_res_enter(hs_net *net)
+{
+    HsResNet &r = net->res;
+    if (r.active) return HS_OK;
+    if (net->mode == 4 && net->step > 0) {
+        uint64_t p = 0;
+        HS_TRY(hs_pending(net, &p));
+        r.ev_bias += p;
+    }
+    r.active = true;
+    return HS_OK;
+}
+
+/* and back: the accumulators of the pipelined windows are filled again */
+static int hs_res_leave(hs_net *net)
+{
+    HsResNet &r = net->res;
+    if (!r.active) return HS_OK;
+    if (net->mode == 4) {
+        for (HGroup &g : net->g)
+            for (int v = 0; v < HS_MAX_VARS; ++v)
+                if (g.acc[v])
+                    HS_HIP(hipMemsetAsync(g.acc[v], 0, hs_rsize(net) * (size_t)g.n * g.nacc, g_rt.stream));
+        if (net->prec == HS_F64)
+            HS_HIP(hs_launch_res_refill<double>((const DPath<double> *)net->dpaths, (int)net->p.size(), net->ctl,
+                                                net->window, g_rt.stream));
+        else
+            HS_HIP(hs_launch_res_refill<float>((const DPath<float> *)net->dpaths, (int)net->p.size(), net->ctl,
+                                               net->window, g_rt.stream));
+        uint64_t p = 0;
+        HS_TRY(hs_pending(net, &p));
+        r.ev_bias -= p;
+    }
+    r.active = false;
+    return HS_OK;
+}
+
+/* steps of one resident launch: bounded, so that a run of any length reports in between */
+#define HS_RES_STEPS 16384
+
+template <typename R>
+static int hs_res_run(hs_net *net, int64_t nsteps, int64_t *left)
+{
+    HsResNet &r = net->res;
+    const HsResArgs<R> &a = hs_res_args<R>(r);
+    HGroup &g = net->g[0];
+    HMon *M = g.smon >= 0 ? &net->m[g.smon] : nullptr;
+    *left = 0;
+    HS_TRY(hs_res_enter(net));
+    const int ms = hs_kernel_model(net, g.model);
+    auto t0 = std::chrono::steady_clock::now();
+    HS_HIP(hipEventRecord(net->ev0, g_rt.stream));
+    const int64_t end = net->step + nsteps;
+    bool known = false; /* info->records is the spike monitor's count */
+    while (net->step < end) {
+        int64_t k = std::min<int64_t>(end - net->step, HS_RES_STEPS);
+        if (M) {
+            /* as many steps as the monitor has room for, whatever spikes */
+            unsigned long long n = r.info->records;
+            if (!known) {
+                HS_HIP(hipMemcpyAsync(&n, M->mn, sizeof(n), hipMemcpyDeviceToHost, g_rt.stream));
+                HS_HIP(hipStreamSynchronize(g_rt.stream));
+            }
+            if ((int64_t)n > M->cap)
+                return hs_fail(HS_ERR_OVERFLOW, "spike monitor overflow: %llu records for capacity %lld", n,
+                               (long long)M->cap);
+            int64_t room = (M->cap - (int64_t)n) / g.n;
+            if (room < std::min<int64_t>(k, 256)) {
+                bool resized = false;
+                HS_TRY(hs_check_spike_monitors(net, std::min<int64_t>(k, 256), &resized));
+                if (resized) HS_TRY(hs_upload_desc(net));
+                room = (M->cap - (int64_t)n) / g.n;
+            }
+            k = std::min(k, std::max<int64_t>(room, 1));
+        }
+        const int64_t wins = (k + a.W - 1) / a.W;
+        if ((int64_t)r.win + wins + 1 > 0xffffffffLL) { /* window numbers start over */
+            HS_HIP(hipMemsetAsync(a.mail, 0, r.mail_bytes, g_rt.stream));
+            r.win = 1;
+        }
+        if (hs_launch_resident<R>(a, (const HsResArgs<R> *)r.dargs, (const DGroup<R> *)net->dgroups, ms,
+                                  net->engine == HS_ENGINE_PLAIN, r.block, net->step, (int)k, r.win,
+                                  g_rt.stream) != hipSuccess) {
+            /* no cooperative launch to be had (another process of this GPU holds
+               them): nothing has been enqueued, the per-step forms take over */
+            (void)hipGetLastError();
+            r.state = -1;
+            *left = end - net->step;
+            return HS_OK;
+        }
+        HS_HIP(hs_launch_res_close<R>(a, (const DGroup<R> *)net->dgroups, r.block, net->step, (int)k, r.info,
+                                      g_rt.stream));
+        r.win += (uint32_t)wins;
+        net->step += k;
+        if (net->step >= end) HS_HIP(hipEventRecord(net->ev1, g_rt.stream));
+        HS_HIP(hipStreamSynchronize(g_rt.stream));
+        known = true;
+        if (r.info->stalled || r.info->base != net->step) {
+            r.state = -2;
+            return hs_fail(HS_ERR_HIP, "resident step loop: a block waited in vain for the others (step %lld of %lld)",
+                           r.info->base, (long long)net->step);
+        }
+    }
+    auto t1 = std::chrono::steady_clock::now();
+    float ms_gpu = 0;
+    HS_HIP(hipEventElapsedTime(&ms_gpu, net->ev0, net->ev1));
+    net->last_gpu_ms = ms_gpu;
+    net->last_wall = std::chrono::duration<double>(t1 - t0).count();
+    net->last_steps = nsteps;
+    net->events = r.info->events - r.ev_bias;
+    net->spikes = r.info->spikes;
+    if (M && (int64_t)r.info->records > M->cap)
+        return hs_fail(HS_ERR_OVERFLOW, "spike monitor overflow: %llu records for capacity %lld", r.info->records,
+                       (long long)M->cap);
+    return HS_OK;
+}
+
 extern "C" int hs_net_run(hs_net *net, int64_t nsteps)
 {
     if (!net) return hs_fail(HS_ERR_ARG, "null net");
     if (nsteps < 0) return hs_fail(HS_ERR_ARG, "negative step count");
     if (net->g.empty()) return hs_fail(HS_ERR_STATE, "network has no groups");
     HS_TRY(hs_prepare_run(net, nsteps));
+    bool resident = false;
+    HS_TRY(hs_res_ready(net, nsteps, &resident));
+    if (net->res.state == -2) return hs_fail(HS_ERR_STATE, "the network's last run was given up");
+    if (resident) {
+        int64_t left = 0;
+        HS_TRY(net->prec == HS_F64 ? hs_res_run<double>(net, nsteps, &left) : hs_res_run<float>(net, nsteps, &left));
+        if (left == 0) return HS_OK;
+        nsteps = left;
+    }
+    HS_TRY(hs_res_leave(net));
+    net->res.asked += nsteps;
     bool have_smon = false;
     for (const HMon &M : net->m) have_smon |= (M.kind == 0);
     const int64_t K = net->opt[2] > 0 ? net->opt[2] : 256;
@@ -2427,7 +2768,7 @@ extern "C" int hs_net_run(hs_net *net, int64_t nsteps)
     HsCtl &c = cbuf[0];
     HS_HIP(hipMemcpyAsync(&c, net->ctl, sizeof(c), hipMemcpyDeviceToHost, g_rt.stream));
     HS_HIP(hipStreamSynchronize(g_rt.stream));
-    net->events = hs_ctl_events(c) - (net->mode == 4 ? c.pending : 0ull);
+    net->events = hs_ctl_events(c) - (net->mode == 4 ? c.pending : 0ull) - net->res.ev_bias;
     net->spikes = hs_ctl_spikes(c);
     if (c.base != net->step) return hs_fail(HS_ERR_STATE, "device step %lld != host step %lld", c.base, (long long)net->step);
     for (const HMon &M : net->m) {

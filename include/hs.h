@@ -450,6 +450,12 @@ int hs_net_set_monitor_interval(hs_net *net, int mid, int every);
  * 11 fast math (FP32 only; 1: the COBA Hodgkin-Huxley update uses the device
  * exponential, reciprocal division and FMA contraction -- faster, not
  * bit-reproducible by the oracle; its error is measured against FP64).
+ * 12 resident step loop (1, the default: a network of one built-in group whose
+ * pathways are scattered and whose neurons and delays fit the chip runs many
+ * steps per launch, its state in registers and LDS, once it is asked for enough
+ * steps to pay for laying its synapses out; the same results, whatever keys 0 to
+ * 10 say; 0: always the per-step forms that they describe, as with key 7).
+ * Key 13 can only be read: 1 if the last run was resident.
  * brian2cuda_amd/autotune.py picks keys 0, 1, 3, 4, 8, 9, 10 by measurement. */
 int hs_net_set_option(hs_net *net, int key, long long value);
 int hs_net_get_option(hs_net *net, int key, long long *value);
@@ -460,8 +466,9 @@ int hs_net_get_option(hs_net *net, int key, long long *value);
 int hs_net_kernel_time(hs_net *net, int kind, double *total_ms, int64_t *launches);
 
 /*
- * Advance nsteps time steps.  Steps run in chunks captured as HIP graphs; no
- * host synchronisation inside a chunk (counts stay on the device).  Pending
+ * Advance nsteps time steps.  Steps run in one launch (the resident loop, key 12)
+ * or in chunks captured as HIP graphs; no host synchronisation inside a chunk
+ * (counts stay on the device).  Pending
  * effects and resets are applied at the end so that state reads see Brian2's
  * post-step state.  Replaces Network::run (network.cu:40-137).
  */
@@ -488,7 +495,7 @@ typedef struct {
     double last_run_wall_s;  /* wall time of the last hs_net_run (host clock) */
     double last_run_gpu_ms;  /* device time of the last run's step chunks (HIP events) */
     int64_t last_run_steps;
-    double launches_per_step; /* kernel launches per simulated step */
+    double launches_per_step; /* kernel launches per simulated step in the network's per-step form */
     int64_t window;           /* steps per update launch (fused form with delays >= 2 steps) */
 } hs_stats;
 int hs_net_stats(hs_net *net, hs_stats *out);

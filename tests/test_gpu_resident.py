@@ -1,0 +1,116 @@
+"""The resident step loop (option 12) at the sizes where it can go wrong, and the
+per-step forms it replaces on small networks: bit for bit against the oracle, and
+against each other when a network changes between them mid-run."""
+import numpy as np
+import pytest
+
+from brian2cuda_amd import networks as nw
+from brian2cuda_amd import runtime as rt
+from test_gpu_networks import ENGINES, _compare
+
+pytestmark = pytest.mark.gpu
+
+
+def _cuba(n, p, delays, seed=3, we=0.3e-3, wi=-1e-3):
+    """n CUBA neurons, random pairs, one weight per pathway, delays drawn from `delays`."""
+    rng = np.random.default_rng(seed)
+    spec = nw.cuba(N=n, seed=seed, monitors=False)
+    ne, paths = max(1, int(0.8 * n)), []
+    for var, w, (lo, hi) in ((1, we, (0, ne)), (2, wi, (ne, n))):
+        pre, post = np.nonzero(rng.random((hi - lo, n)) < p)
+        paths.append(nw.PathSpec(0, 0, var, (pre + lo).astype(np.int32), post.astype(np.int32),
+                                 delay_steps=rng.choice(delays, pre.size).astype(np.int32), wmode=0, wscalar=w))
+    spec.paths = paths
+    spec.spike_monitors = [0]
+    spec.state_monitors = [(0, 0, 0, min(n, 5))]
+    return spec
+
+
+def _was_resident(net):
+    return net.get_option(rt.OPT_WAS_RESIDENT) == 1
+
+
+@pytest.mark.parametrize("engine,sem", ENGINES)
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n,p,delays", [(1, 1.0, [1]), (2, 1.0, [0]), (63, 0.5, [1]), (64, 0.5, [0, 3]), (65, 0.3, [2]),
+                                        (513, 0.1, [1, 2, 3, 40]), (1000, 0.05, [7]), (4097, 0.01, [1]),
+                                        (5000, 0.02, [9, 60])])
+def test_sizes_and_delays(hs, oracle_lib, n, p, delays, prec, engine, sem):
+    """One block and many, ragged last blocks and waves; windows of 1 to 8 steps and
+    runs that end inside one; delays shorter and longer than a run."""
+    net, _ = _compare(_cuba(n, p, delays), prec, engine, sem, None, oracle_lib, chunks=[20, 1, 11, 3, 300])
+    assert _was_resident(net)
+
+
+@pytest.mark.parametrize("engine,sem", ENGINES)
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n,delays", [(1000, [1]), (1000, [3]), (700, [0, 1, 2, 30])])
+def test_everyone_fires(hs, oracle_lib, n, delays, prec, engine, sem):
+    """All neurons fire in one step: lines of more spikes than a header or a polling
+    thread takes, buckets of the plain form that overflow and are delivered from the
+    spikes of this launch or of the one before."""
+    spec = _cuba(n, 0.5, delays, we=1e-6, wi=-1e-6)
+    spec.groups[0].init[0] = np.full(n, -49.5e-3)
+    for chunks in ([60, 60], [12, 2, 1, 1, 50]):
+        net, ref = _compare(spec, prec, engine, sem, None, oracle_lib, chunks=chunks)
+        assert _was_resident(net) and ref.events > 0.4 * n * n
+
+
+@pytest.mark.parametrize("opts", [{}, {9: 1}, {9: 1, 4: 2}])
+@pytest.mark.parametrize("engine,sem", ENGINES)
+@pytest.mark.parametrize("spec", ["brunel", "cuba", "cobahh"])
+def test_changes_between_the_forms(hs, oracle_lib, spec, engine, sem, opts):
+    """A network that leaves the resident loop and comes back gives the oracle's bits
+    throughout, events in flight included."""
+    spec = {"brunel": lambda: nw.brunel(N=2000, K=200, seed=4, monitors=True), "cuba": lambda: nw.cuba(N=1500, seed=5),
+            "cobahh": lambda: nw.cobahh(N=600, seed=6)}[spec]()
+    for prec in (64, 32):
+        net, smon, _ = nw.build_hs(spec, prec, engine, options=opts)
+        ref, rsmon, _ = oracle_lib.build_ref(spec, prec, sem)
+        for k, on in ((40, 0), (300, 1), (33, 0), (1, 1), (2, 0), (250, 1), (200, 0)):
+            net.set_option(rt.OPT_RESIDENT, on)
+            net.run(k)
+            ref.run(k)
+            assert _was_resident(net) == bool(on)
+            assert net.stats()["events"] == ref.events
+            assert np.array_equal(net.get_state(0, 0), ref.get_state(0, 0), equal_nan=True)
+        gi, gt = net.spikes(smon[0])
+        ri, rtt = ref.spikes(rsmon[0])
+        assert len(gi) > 100 and np.array_equal(gi, ri) and np.array_equal(gt, rtt)
+        net.close()
+
+
+def test_layout_waits_for_enough_steps(hs):
+    """Many synapses and few steps: the per-step form runs until the steps asked for pay for the layout."""
+    spec = nw.brunel(N=4000, K=1000, seed=2, device_connect=True)  # 4e6 synapses: 90 steps
+    net, _, _ = nw.build_hs(spec, 32, "fused")
+    seen = []
+    for _ in range(4):
+        net.run(40)
+        seen.append(_was_resident(net))
+    assert seen == [False, False, True, True]
+    net.close()
+
+
+def test_refuses_nothing_and_leaves_the_rest_alone(hs, oracle_lib):
+    """Networks outside the loop's geometry keep running in the per-step forms: more
+    neurons than the chip's blocks own, sums that do not fit LDS, several groups."""
+    big = nw.brunel(N=140_000, K=10, seed=1, device_connect=True)
+    wide = nw.brunel(N=100_000, K=20, seed=1, device_connect=True)
+    for spec, prec, engine in ((big, 32, "fused"), (wide, 64, "fused"), (nw.code_mix(N=400, monitors=False), 64, "plain")):
+        net, _, _ = nw.build_hs(spec, prec, engine)
+        net.run(100)
+        assert not _was_resident(net)
+        net.close()
+
+
+@pytest.mark.parametrize("opts", [{}, {9: 1}, {4: 3}, {9: 1, 4: 2, 0: 64, 1: 768, 8: 768}, {0: 128, 1: 512, 10: 256},
+                                  {2: 0}])
+@pytest.mark.parametrize("engine,sem", ENGINES)
+@pytest.mark.parametrize("prec", [64, 32])
+def test_per_step_forms_on_small_networks(hs, oracle_lib, prec, engine, sem, opts):
+    """The update, delivery, fused and window kernels, which larger networks run."""
+    opts = {**opts, rt.OPT_RESIDENT: 0}
+    for spec in (nw.brunel(N=2500, K=250, seed=6, monitors=True), nw.cuba(N=1500, seed=5), nw.cobahh(N=600, seed=6)):
+        net, _ = _compare(spec, prec, engine, sem, None, oracle_lib, options=opts, chunks=[7, 300, 93])
+        assert not _was_resident(net)
