@@ -41,10 +41,10 @@ HIPCC_FLAGS = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-result",
 ]
 
-# hs_resident.hip: the polynomials' 64-bit constants stay where they are used (two
+# hs_resident.hip, hs_hines.hip: the polynomials' 64-bit constants stay where they are used (two
 # scalar moves) instead of being hoisted out of the step loop, where they exceed
 # the scalar registers and are spilled (254 -> 76 spills in the FP64 noise model)
-SOURCE_FLAGS = {"hs_resident.hip": ["-mllvm", "-disable-machine-licm"]}
+SOURCE_FLAGS = {f: ["-mllvm", "-disable-machine-licm"] for f in ("hs_resident.hip", "hs_hines.hip")}
 
 
 def hipcc_path():

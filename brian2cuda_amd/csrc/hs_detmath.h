@@ -48,11 +48,9 @@
 #define HS_LN2F_LO 3.194618329871446e-05f
 #define HS_LOG2EF 1.44269504f
 
-HS_HD double hs_exp(double x)
+/* for -708 <= x <= 709 */
+HS_HD double hs_exp_core(double x)
 {
-    /* keep 2^k in the normal range; NaN falls through the comparisons */
-    if (x > 709.0) x = 709.0;
-    if (x < -708.0) x = -708.0;
     double kd = floor(x * HS_LOG2E + 0.5);
     double r = (x - kd * HS_LN2_HI) - kd * HS_LN2_LO;
     double p = 1.6059043836821613e-10;           /* 1/13! */
@@ -72,10 +70,17 @@ HS_HD double hs_exp(double x)
     return ldexp(p, (int)kd);
 }
 
-HS_HD float hs_expf(float x)
+HS_HD double hs_exp(double x)
 {
-    if (x > 88.0f) x = 88.0f;
-    if (x < -87.0f) x = -87.0f;
+    /* keep 2^k in the normal range; NaN falls through the comparisons */
+    if (x > 709.0) x = 709.0;
+    if (x < -708.0) x = -708.0;
+    return hs_exp_core(x);
+}
+
+/* for -87 <= x <= 88 */
+HS_HD float hs_expf_core(float x)
+{
     float kf = floorf(x * HS_LOG2EF + 0.5f);
     float r = (x - kf * HS_LN2F_HI) - kf * HS_LN2F_LO;
     float p = 0.00019841270113829523f;           /* 1/7! */
@@ -87,6 +92,13 @@ HS_HD float hs_expf(float x)
     p = 1.0f + r * p;
     p = 1.0f + r * p;
     return ldexpf(p, (int)kf);
+}
+
+HS_HD float hs_expf(float x)
+{
+    if (x > 88.0f) x = 88.0f;
+    if (x < -87.0f) x = -87.0f;
+    return hs_expf_core(x);
 }
 
 /* natural log for finite x > 0 (callers guarantee it: uniforms in (0, 1]) */

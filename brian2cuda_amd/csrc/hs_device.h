@@ -107,12 +107,14 @@ __device__ __forceinline__ int hs_wrap(int x, int m)
 #define HS_SFX(name) name##_f32fast
 #define HS_EXP __expf
 #define HS_DIV(a, b) ((a) * __builtin_amdgcn_rcpf(b))
+#define HS_DIVC HS_DIV
 #define HS_FAST_CONTRACT _Pragma("clang fp contract(fast)")
 #include "hs_model_body.inc"
 #undef R
 #undef HS_SFX
 #undef HS_EXP
 #undef HS_DIV
+#undef HS_DIVC
 #undef HS_FAST_CONTRACT
 #pragma pop_macro("HS_HD")
 

@@ -10,6 +10,7 @@
 
 /* the exact instances: IEEE division, no contraction (the numerical contract) */
 #define HS_DIV(a, b) ((a) / (b))
+#define HS_DIVC(a, c) ((a) / (c))
 #define HS_FAST_CONTRACT
 
 #define R double
@@ -28,6 +29,7 @@
 #undef HS_SFX
 #undef HS_EXP
 #undef HS_DIV
+#undef HS_DIVC
 #undef HS_FAST_CONTRACT
 
 /*
