@@ -2400,6 +2400,8 @@ static int hs_check_spike_monitors(hs_net *net, int64_t k, bool *resized)
 
 #define HS_RES_MIN_STEPS 10
 #define HS_RES_SYN_PER_STEP 50000
+#define HS_RES_BIG 1000000
+#define HS_RES_FIRST_STEPS 1500
 
 /* LDS a block may use: the compute unit's 160 KiB, with a margin */
 #define HS_RES_LDS (156 * 1024)
@@ -2551,7 +2553,14 @@ static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use)
            forms, and one that goes on changes over */
         int64_t total = 0;
         for (const HPath &P : net->p) total += P.nsyn;
-        if (r.asked + nsteps < HS_RES_MIN_STEPS + total / HS_RES_SYN_PER_STEP) return HS_OK;
+        int64_t worth = HS_RES_MIN_STEPS + total / HS_RES_SYN_PER_STEP;
+        /* beyond HS_RES_BIG synapses the allocations and their release are another 2 ms: a
+           first run has to earn them by itself (a script of one run: 20,000 neurons, 4e6
+           synapses, 100 steps, built and taken down, 12.3 ms in the per-step forms and
+           14.1 resident; 50,000, 1.5e7, 380 steps 5.4 and 7.1; 20,000, 1.2e7, 300 steps
+           3.8 and 4.5); a network that is run again goes on */
+        if (total > HS_RES_BIG && r.asked == 0) worth += HS_RES_FIRST_STEPS;
+        if (r.asked + nsteps < worth) return HS_OK;
         HS_TRY(hs_res_layout<R>(net));
         if (r.state < 0) return HS_OK;
     }
