@@ -2419,8 +2419,6 @@ static bool hs_res_geometry(hs_net *net)
         return false;
     const HGroup &g = net->g[0];
     if (g.model != HS_MODEL_LIF_CUBA && g.model != HS_MODEL_LIF_NOISE && g.model != HS_MODEL_HH_COBA) return false;
-    for (const HMon &M : net->m)
-        if (M.kind == 3) return false;
     int64_t total = 0;
     int dmin = 1 << 30, dmax = 0;
     for (int v = 0; v < HS_MAX_VARS; ++v) a.plane[v] = -1;
@@ -2542,6 +2540,10 @@ static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use)
     HsResNet &r = net->res;
     *use = false;
     if (r.state < 0 || !net->opt[12] || net->opt[7] || nsteps == 0) return HS_OK;
+    /* asked before every run: a plain network takes synapse StateMonitors between runs,
+       and only the per-step forms record them */
+    for (const HMon &M : net->m)
+        if (M.kind == 3) return HS_OK;
     if (r.state == 0) {
         if (!hs_res_geometry<R>(net)) {
             r.state = -1;

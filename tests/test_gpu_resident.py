@@ -114,3 +114,30 @@ def test_per_step_forms_on_small_networks(hs, oracle_lib, prec, engine, sem, opt
     for spec in (nw.brunel(N=2500, K=250, seed=6, monitors=True), nw.cuba(N=1500, seed=5), nw.cobahh(N=600, seed=6)):
         net, _ = _compare(spec, prec, engine, sem, None, oracle_lib, options=opts, chunks=[7, 300, 93])
         assert not _was_resident(net)
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("engine,sem,delay", [("plain", 0, 1), ("plain", 0, 0), ("fused", 1, 0)])
+def test_synapse_monitor_between_runs(hs, oracle_lib, engine, sem, delay, prec):
+    """A synapse StateMonitor added after a resident run records every step that
+    follows: the network goes on in the per-step form, with the oracle's bits."""
+    spec = _cuba(300, 0.1, [delay])
+    P = spec.paths[0]
+    P.wmode, P.weights = rt.HS_W_SYNAPSE, np.full(P.nsyn, P.wscalar)
+    net, smon, _ = nw.build_hs(spec, prec, engine)
+    ref, rsmon, _ = oracle_lib.build_ref(spec, prec, sem)
+    net.run(60)
+    assert _was_resident(net)
+    which = np.array([5, 0, P.nsyn - 1, 7], np.int32)
+    mid = net.add_synapse_monitor(0, rt.HS_SYN_W, which)
+    net.run(30)
+    net.run(31)
+    assert not _was_resident(net)
+    w = net.synapse_var(0, rt.HS_SYN_W)[which]
+    assert w.min() > 0
+    np.testing.assert_array_equal(net.state_monitor(mid, which.size), np.tile(w, (61, 1)))
+    ref.run(121)
+    assert net.stats()["events"] == ref.events
+    for a, b in zip(net.spikes(smon[0]), ref.spikes(rsmon[0])):
+        np.testing.assert_array_equal(a, b)
+    net.close()
