@@ -49,7 +49,8 @@
  * rates is the compiler's sequence (v_rcp, two Newton steps, quotient, residual
  * correction) without v_div_scale and v_div_fixup, which only act outside the
  * exponent range that the constants (checked when the batch is created) and the
- * potentials (checked every step, a step outside takes the IEEE division) stay in;
+ * potentials and conductances (checked every step, a step outside takes the IEEE
+ * division) stay in;
  * a division by a constant c is x*(1/c) and one residual correction, exact because
  * 1/c rounded is within half an ulp's relative error of 1/c for these c; exp skips
  * its clamps.
@@ -74,6 +75,9 @@
 #define HS_HINES_VLO (-0.1)
 #define HS_HINES_VHI 0.2
 #define HS_HINES_DTMAX 7e-5
+/* conductance densities (S/m2) that leave the rows' pivots to their constants: gates may be
+   set to anything, and a pivot of 0 or infinity takes the IEEE division */
+#define HS_HINES_GMAX 1e30
 
 template <typename R>
 struct HinesDesc {
@@ -526,7 +530,7 @@ __global__ __launch_bounds__(1024) void hs_k_hines(const HinesDesc<R> d, int nst
                 const double I0 = (double)i0 + iext;
                 L.row[j].a = ab1 - (double)gt;
                 L.row[j].v = -(cdt * v) - I0;
-                wild |= !(v > HS_HINES_VLO && v < HS_HINES_VHI);
+                wild |= !(v > HS_HINES_VLO && v < HS_HINES_VHI && gt >= 0 && gt < (R)HS_HINES_GMAX);
             }
         }
         if (step == nsteps) break;

@@ -54,7 +54,7 @@ def test_trees_per_unit(hs, n_trees):
 
 
 @pytest.mark.parametrize("prec", [64, 32])
-@pytest.mark.parametrize("kind", ["potential", "step", "weak"])
+@pytest.mark.parametrize("kind", ["potential", "step", "weak", "gates", "negative", "nan"])
 def test_outside_the_short_forms(hs, kind, prec):
     tb = _combs([4, 3, 200], n_trees=3, dt=0.1e-3 if kind == "step" else 0.025e-3, l=3e-3 if kind == "weak" else 30e-6)
     if kind == "potential":
@@ -62,4 +62,12 @@ def test_outside_the_short_forms(hs, kind, prec):
         tb.init[0][tb.n_comp // 2] = -0.2
     if kind == "weak": # each compartment sees about 1e-6 of its neighbour: 200 of them reach below the smallest double
         tb.init[0][:] = 0
+    if kind == "gates": # two conductances whose sum leaves the exponent range, their currents do not: a row divides by infinity
+        most = 1.6e308 if prec == 64 else 3e38
+        for i in (5, tb.n_comp // 2):
+            tb.init[1][i], tb.init[2][i] = (most / tb.chan[2]) ** (1 / 3), (0.8 * most / tb.chan[4]) ** 0.25
+    if kind == "negative": # a diagonal of either sign
+        tb.init[3][9:12] = [-1e3, -0.05, -1e-3]
+    if kind == "nan":
+        tb.init[1][5] = np.nan
     _check(tb, prec, 40)
