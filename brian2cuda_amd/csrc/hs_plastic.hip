@@ -12,15 +12,27 @@
  * only writes synapse variables).
  *
  * on_pre (step T): for each delay slot d, the spikes of step T - dmin - d; block
- * b takes slots b, b + grid, ...  The threads take first the slot's spikes, 256 at a
- * time, each finding its bundle, and then the synapses of these bundles laid end to
- * end, 256 at a time.  A synapse sits in one bundle and a neuron spikes at most once
- * a step, so no two threads touch the same synapse; the target effect is a
- * hardware FP atomic (other delays and pathways reach the target too), and the
- * effects of 256 synapses on one target are added by one thread, in the order of the
- * spikes.  A step is bound by its chain of dependent loads (count, spike, bundle,
- * synapse, target: about 5 us), so the spikes share one instead of having one each:
- * 10,000 Poisson inputs with 15 spikes a step on 10 neurons, on_pre 12.6 -> 7.3 us.
+ * b takes slots b, b + grid, ...  A synapse sits in one bundle and a neuron spikes at
+ * most once a step, so no two threads touch the same synapse; the target effect is a
+ * hardware FP atomic (several synapses share a target).  A spike costs a chain of
+ * dependent loads (count, spike, bundle, synapse, target), so beyond HS_STDP_FEW
+ * spikes the threads find the bundles of 256 spikes at once, and then
+ *   mean bundle up to HS_STDP_SHARE synapses: they take the synapses laid end to end,
+ *     256 at a time; the effects on one target are added by one thread, in the order
+ *     of the spikes, which it finds by comparing the round's targets (0.1 us a
+ *     synapse);
+ *   longer bundles: one after another, each by all threads (0.6 us a spike).
+ * Measured, us a step of a network (update, on_pre, on_post; FP64) with a chain per
+ * spike -> now, of it all synapses end to end and all bundles one after another:
+ *   spikes  synapses each
+ *     1.5      1           9.8 -> 10.0  (10.5, 10.6)
+ *    15        1          19.6 -> 12.7  (12.9, 18.1)
+ *    15        6          23.6 -> 20.8  (20.3, 22.0)
+ *    15        8          23.6 -> 22.1  (23.3, 22.2)
+ *   100        4         103.7 -> 49.5  (50.3, 82.9)
+ *   100        8         103.9 -> 85.8  (88.8, 83.5)
+ *    15     1000          81.4 -> 62.4  (1000, 68.1)
+ *    10    10000           638 -> 430   (6510, 431)
  * on_post (step T): the target group's spikes of step T, block-strided; the
  * threads take that neuron's synapses (qsyn).  Launched after on_pre: Brian2
  * runs the pre pathway (order -1) before the post pathway (order +1) within the
@@ -66,6 +78,8 @@ template <> struct HsStdp<float> {
 };
 
 #define HS_STDP_BLOCK 256
+#define HS_STDP_FEW 2   /* spikes up to which the scans cost more than their chains: 1 us a step */
+#define HS_STDP_SHARE 6 /* synapses per spike: the two forms meet between 6 and 8 */
 
 /* exclusive prefix sum over the block; *total: of all threads.  scratch: one int per
    wave, free again after the next barrier of the caller */
@@ -100,6 +114,34 @@ __device__ __forceinline__ int hs_stdp_find(const int *at, int x)
     return lo;
 }
 
+/* the on_pre code of synapse q at step T; returns the effect on its target */
+template <typename R>
+__device__ __forceinline__ R hs_stdp_synapse(const DPath<R> &p, int q, long long T, const R *sk)
+{
+    const long long n = T - (long long)p.lastup[q];
+    const R fa = HsStdp<R>::decay(n, p.dt, p.taupre);
+    const R fb = HsStdp<R>::decay(n, p.dt, p.taupost);
+    R w = p.wm[q], a = p.apre[q], b = p.apost[q];
+    const R e = HsStdp<R>::pre(&w, &a, &b, fa, fb, sk);
+    p.wm[q] = w;
+    p.apre[q] = a;
+    p.apost[q] = b;
+    p.lastup[q] = (int32_t)T;
+    return e;
+}
+
+/* synapses [q0, q1) of a bundle by the threads of the block */
+template <typename R>
+__device__ __forceinline__ void hs_stdp_bundle(const DPath<R> &p, int q0, int q1, long long T, const R *sk, R *tgt,
+                                               unsigned long long *ev)
+{
+    for (int q = q0 + (int)threadIdx.x; q < q1; q += HS_STDP_BLOCK) {
+        const int j = p.post[q];
+        hs_atomic_add(tgt + j, hs_stdp_synapse(p, q, T, sk));
+        ++*ev;
+    }
+}
+
 template <typename R>
 __global__ __launch_bounds__(HS_STDP_BLOCK) void hs_k_stdp_pre(const DPath<R> *paths, int np, HsCtl *ctl, int koff)
 {
@@ -122,37 +164,49 @@ __global__ __launch_bounds__(HS_STDP_BLOCK) void hs_k_stdp_pre(const DPath<R> *p
             const long long ts = T - p.dmin - d; /* emission step of the bundles due now */
             if (ts < 0) continue;
             const long long slot = hs_mod(ts, p.Q);
+            const int32_t *const hist = p.hist + slot * p.nsub * p.subcap;
             for (int sl0 = 0; sl0 < p.nsub; sl0 += HS_STDP_BLOCK) { /* the lists of the slot */
-                const int sl = sl0 + tid;
                 int nspk, nsyn;
-                s_list[tid] = hs_stdp_scan(sl < p.nsub ? p.hist_cnt[(slot * p.nsub + sl) * p.cstride] : 0, s_sum[0], &nspk);
-                __syncthreads();
+                if (p.nsub == 1) {
+                    nspk = p.hist_cnt[slot * p.cstride];
+                    if (nspk <= HS_STDP_FEW) {
+                        for (int k = 0; k < nspk; ++k) {
+                            const long long row = (long long)hist[k] * p.D + d;
+                            hs_stdp_bundle(p, p.bstart[row], p.bstart[row + 1], T, sk, tgt, &ev);
+                        }
+                        continue;
+                    }
+                } else {
+                    const int sl = sl0 + tid;
+                    s_list[tid] = hs_stdp_scan(sl < p.nsub ? p.hist_cnt[(slot * p.nsub + sl) * p.cstride] : 0, s_sum[0], &nspk);
+                    __syncthreads();
+                }
                 for (int k0 = 0; k0 < nspk; k0 += HS_STDP_BLOCK) { /* their spikes */
                     int from = 0, size = 0;
                     if (k0 + tid < nspk) {
-                        const int l = hs_stdp_find(s_list, k0 + tid);
-                        const long long i = p.hist[slot * p.nsub * p.subcap + (long long)(sl0 + l) * p.subcap + (k0 + tid - s_list[l])];
+                        const int l = p.nsub == 1 ? 0 : hs_stdp_find(s_list, k0 + tid), at = p.nsub == 1 ? 0 : s_list[l];
+                        const long long i = hist[(long long)(sl0 + l) * p.subcap + (k0 + tid - at)];
                         from = p.bstart[i * p.D + d];
                         size = p.bstart[i * p.D + d + 1] - from;
                     }
                     s_at[tid] = hs_stdp_scan(size, s_sum[1], &nsyn);
                     s_from[tid] = from;
                     __syncthreads();
+                    const int m = min(nspk - k0, HS_STDP_BLOCK);
+                    if (nsyn > HS_STDP_SHARE * m) { /* a bundle after the other */
+                        for (int k = 0; k < m; ++k)
+                            hs_stdp_bundle(p, s_from[k], s_from[k] + (k + 1 < m ? s_at[k + 1] : nsyn) - s_at[k], T, sk, tgt,
+                                           &ev);
+                        __syncthreads();
+                        continue;
+                    }
                     for (int m0 = 0; m0 < nsyn; m0 += HS_STDP_BLOCK) { /* their synapses */
                         const int n = min(nsyn - m0, HS_STDP_BLOCK);
                         int j = -1;
                         if (tid < n) {
                             const int k = hs_stdp_find(s_at, m0 + tid), q = s_from[k] + (m0 + tid - s_at[k]);
-                            const long long past = T - (long long)p.lastup[q];
-                            R w = p.wm[q], a = p.apre[q], b = p.apost[q];
                             j = p.post[q];
-                            const R fa = HsStdp<R>::decay(past, p.dt, p.taupre);
-                            const R fb = HsStdp<R>::decay(past, p.dt, p.taupost);
-                            s_eff[tid] = HsStdp<R>::pre(&w, &a, &b, fa, fb, sk);
-                            p.wm[q] = w;
-                            p.apre[q] = a;
-                            p.apost[q] = b;
-                            p.lastup[q] = (int32_t)T;
+                            s_eff[tid] = hs_stdp_synapse(p, q, T, sk);
                             ev++;
                         }
                         s_post[tid] = j;
