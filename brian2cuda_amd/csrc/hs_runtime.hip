@@ -2632,8 +2632,9 @@ static int hs_res_leave(hs_net *net)
 /* steps of one resident launch: bounded, so that a run of any length reports in between */
 #define HS_RES_STEPS 16384
 
+/* t0: when the run began */
 template <typename R>
-static int hs_res_run(hs_net *net, int64_t nsteps, int64_t *left)
+static int hs_res_run(hs_net *net, int64_t nsteps, std::chrono::steady_clock::time_point t0, int64_t *left)
 {
     HsResNet &r = net->res;
     const HsResArgs<R> &a = hs_res_args<R>(r);
@@ -2642,7 +2643,6 @@ static int hs_res_run(hs_net *net, int64_t nsteps, int64_t *left)
     *left = 0;
     HS_TRY(hs_res_enter(net));
     const int ms = hs_kernel_model(net, g.model);
-    auto t0 = std::chrono::steady_clock::now();
     HS_HIP(hipEventRecord(net->ev0, g_rt.stream));
     const int64_t end = net->step + nsteps;
     bool known = false; /* info->records is the spike monitor's count */
@@ -2715,12 +2715,16 @@ extern "C" int hs_net_run(hs_net *net, int64_t nsteps)
     if (nsteps < 0) return hs_fail(HS_ERR_ARG, "negative step count");
     if (net->g.empty()) return hs_fail(HS_ERR_STATE, "network has no groups");
     HS_TRY(hs_prepare_run(net, nsteps));
+    /* the run's time, with the synapses' layout or the graphs that hs_net_prepare did not make */
+    const auto t0 = std::chrono::steady_clock::now();
+    const int64_t asked = nsteps;
     bool resident = false;
     HS_TRY(hs_res_ready(net, nsteps, &resident));
     if (net->res.state == -2) return hs_fail(HS_ERR_STATE, "the network's last run was given up");
     if (resident) {
         int64_t left = 0;
-        HS_TRY(net->prec == HS_F64 ? hs_res_run<double>(net, nsteps, &left) : hs_res_run<float>(net, nsteps, &left));
+        HS_TRY(net->prec == HS_F64 ? hs_res_run<double>(net, nsteps, t0, &left)
+                                   : hs_res_run<float>(net, nsteps, t0, &left));
         if (left == 0) return HS_OK;
         nsteps = left;
     }
@@ -2729,8 +2733,7 @@ extern "C" int hs_net_run(hs_net *net, int64_t nsteps)
     bool have_smon = false;
     for (const HMon &M : net->m) have_smon |= (M.kind == 0);
     const int64_t K = net->opt[2] > 0 ? net->opt[2] : 256;
-    auto t0 = std::chrono::steady_clock::now();
-    HS_HIP(hipEventRecord(net->ev0, g_rt.stream));
+    if (!resident) HS_HIP(hipEventRecord(net->ev0, g_rt.stream)); /* else where the resident steps began */
     int64_t done = 0;
     while (done < nsteps) {
         const int64_t k = std::min<int64_t>(K, nsteps - done);
@@ -2773,7 +2776,7 @@ extern "C" int hs_net_run(hs_net *net, int64_t nsteps)
     HS_HIP(hipEventElapsedTime(&ms, net->ev0, net->ev1));
     net->last_gpu_ms = ms;
     net->last_wall = std::chrono::duration<double>(t1 - t0).count();
-    net->last_steps = nsteps;
+    net->last_steps = asked;
     net->step += nsteps;
     std::vector<HsCtl> cbuf(1);
     HsCtl &c = cbuf[0];

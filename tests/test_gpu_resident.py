@@ -141,3 +141,19 @@ def test_synapse_monitor_between_runs(hs, oracle_lib, engine, sem, delay, prec):
     for a, b in zip(net.spikes(smon[0]), ref.spikes(rsmon[0])):
         np.testing.assert_array_equal(a, b)
     net.close()
+
+
+def test_run_time_counts_the_layout(hs):
+    """A run that lays the synapses out takes that long: its time is not that of a run after prepare."""
+    spec, wall = nw.cuba(N=16000, p=0.003, monitors=False), {}  # 7.7e5 synapses
+    for prepared in (False, True):
+        for _ in range(6):
+            net, _, _ = nw.build_hs(spec, 32, "fused")
+            if prepared:
+                net.prepare(40)
+            net.run(40)
+            s = net.stats()
+            assert _was_resident(net) and s["last_run_steps"] == 40
+            wall[prepared] = min(wall.get(prepared, 1.0), s["last_run_wall_s"])
+            net.close()
+    assert wall[False] > 1.5 * wall[True]
