@@ -9,7 +9,10 @@ time by a margin.  Results are cached in a JSON file keyed by the device and a
 signature of the network, so a second call costs nothing.
 
 The options only change launch shapes and the order of floating-point
-additions inside atomics; bit-exact tests run with tuned options too.
+additions inside atomics; bit-exact tests run with tuned options too.  They
+belong to the per-step forms, so these are what is timed (OPT_RESIDENT 0): a
+network that runs in the resident step loop takes its options into account only
+in the runs that are too short to change over to it.
 
 Replaces the fixed launch policies of the reference: threads per bundle and
 blocks chosen from the bundle sizes (brian2cuda/templates/synapses.cu:171-322),
@@ -42,10 +45,11 @@ def candidate_space(n_cu, engine):
 
 
 def signature(spec, precision, engine, device_name):
+    """cache key of what was timed (entries without "per-step" timed the resident loop)"""
     groups = ";".join(f"{g.model}:{g.n}" for g in spec.groups)
     paths = ";".join(f"{p.src}>{p.tgt}:{p.nsyn}:{p.scalar_delay if p.delay_steps is None else 'd'}"
                      for p in spec.paths)
-    return f"{device_name}|{precision}|{engine}|{spec.name}|{groups}|{paths}"
+    return f"per-step|{device_name}|{precision}|{engine}|{spec.name}|{groups}|{paths}"
 
 
 def tune_forms(space, measure, form_key, rounds=3, margin=0.005, log=None):
@@ -98,10 +102,10 @@ def coordinate_descent(space, measure, rounds=3, margin=0.005, log=None):
 
 
 def measure_us_per_step(spec, precision, engine, options, steps, warmup, build=None):
-    """µs per step of a fresh network with `options`, timed by the runtime's
-    own clock around hs_net_run (warm-up steps first)."""
+    """µs per step of a fresh network with `options` in the per-step forms, timed
+    by the runtime's own clock around hs_net_run (warm-up steps first)."""
     from . import networks as nw
-    net, _, _ = (build or nw.build_hs)(spec, precision, engine, options=options)
+    net, _, _ = (build or nw.build_hs)(spec, precision, engine, options={**options, rt.OPT_RESIDENT: 0})
     try:
         net.run(warmup)
         net.run(steps)

@@ -456,7 +456,8 @@ int hs_net_set_monitor_interval(hs_net *net, int mid, int every);
  * steps to pay for laying its synapses out; the same results, whatever keys 0 to
  * 10 say; 0: always the per-step forms that they describe, as with key 7).
  * Key 13 can only be read: 1 if the last run was resident.
- * brian2cuda_amd/autotune.py picks keys 0, 1, 3, 4, 8, 9, 10 by measurement. */
+ * brian2cuda_amd/autotune.py picks keys 0, 1, 3, 4, 8, 9, 10 by measurement in the
+ * per-step forms, the only ones that they act on. */
 int hs_net_set_option(hs_net *net, int key, long long value);
 int hs_net_get_option(hs_net *net, int key, long long *value);
 /* With option 7 on: device time and launch count, summed over the runs since

@@ -3,6 +3,7 @@ import json
 
 from brian2cuda_amd import autotune as at
 from brian2cuda_amd import networks as nw
+from brian2cuda_amd import runtime as rt
 
 
 def test_coordinate_descent_finds_the_separable_minimum():
@@ -60,3 +61,28 @@ def test_cache_write_failure_is_not_fatal(tmp_path, monkeypatch):
                        log=logs.append)
     assert opts == {}
     assert any("cache not written" in m for m in logs)
+
+
+def test_measures_the_per_step_forms():
+    """The options act in the per-step forms alone: the networks that are timed stay out of the resident loop, and a
+    cache written while they did not is not read."""
+    seen = []
+
+    class Net:
+        def run(self, n):
+            seen.append(n)
+
+        def stats(self):
+            return {"last_run_wall_s": 2.0}
+
+        def close(self):
+            seen.append("closed")
+
+    def build(spec, precision, engine, options=None):
+        seen.append(options)
+        return Net(), [], []
+
+    spec = nw.cuba(N=500, seed=1)
+    assert at.measure_us_per_step(spec, 32, "fused", {rt.OPT_UPDATE_BLOCK: 64}, 400, 100, build) == 5000.0
+    assert seen == [{rt.OPT_UPDATE_BLOCK: 64, rt.OPT_RESIDENT: 0}, 100, 400, "closed"]
+    assert at.signature(spec, 32, "fused", "gfx950").startswith("per-step|")
