@@ -7,17 +7,20 @@ import pytest
 
 from brian2cuda_amd import _lib, autotune as at
 from brian2cuda_amd import networks as nw
+from brian2cuda_amd import runtime as rt
 
 pytestmark = pytest.mark.gpu
 
 
 def _same_as_oracle(spec, prec, engine, sem, options, oracle_lib, steps=400):
-    net, sm, _ = nw.build_hs(spec, prec, engine, options=options)
+    """in the per-step forms, which the options shape"""
+    net, sm, _ = nw.build_hs(spec, prec, engine, options={**options, rt.OPT_RESIDENT: 0})
     ref, rsm, _ = oracle_lib.build_ref(spec, prec, sem)
     net.run(steps)
     ref.run(steps)
     gi, gt = net.spikes(sm[0])
     ri, rt_ = ref.spikes(rsm[0])
+    assert net.get_option(rt.OPT_WAS_RESIDENT) == 0
     ok = np.array_equal(gi, ri) and np.array_equal(gt, rt_) and net.stats()["events"] == ref.events
     ok = ok and np.array_equal(net.get_state(0, 0), ref.get_state(0, 0))
     net.close()

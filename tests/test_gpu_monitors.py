@@ -16,7 +16,8 @@ IDX = np.array([3999, 0, 17, 2500, 1234, 3], np.int32)
 
 
 @pytest.mark.parametrize("prec", [64, 32])
-@pytest.mark.parametrize("engine,sem,opts", [("plain", 0, {}), ("fused", 1, {}), ("fused", 1, {9: 1})])
+@pytest.mark.parametrize("engine,sem,opts", [("plain", 0, {}), ("fused", 1, {}), ("plain", 0, {12: 0}),
+                                             ("fused", 1, {12: 0}), ("fused", 1, {9: 1, 12: 0})])
 def test_indexed_interval_monitors_vs_oracle(hs, oracle_lib, prec, engine, sem, opts):
     spec = nw.cuba(N=4000, seed=11, record=0)
     spec.state_monitors = [nw.StateMon(0, 0, IDX, every=10), nw.StateMon(0, 1, np.arange(50)[::-1], every=1),

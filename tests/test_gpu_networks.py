@@ -10,14 +10,20 @@ import numpy as np
 import pytest
 
 from brian2cuda_amd import networks as nw
+from brian2cuda_amd import runtime as hsrt
 
 pytestmark = pytest.mark.gpu
 
 ENGINES = [("plain", 0), ("fused", 1)]
 
 
+def _per_step(options):
+    """Options that shape launches or choose a form belong to the per-step forms: the resident loop would not see them."""
+    return {hsrt.OPT_RESIDENT: 0, **options} if options else options
+
+
 def _compare(spec, prec, engine, sem, steps, oracle_lib, options=None, chunks=None):
-    net, smon, stmon = nw.build_hs(spec, prec, engine, options=options)
+    net, smon, stmon = nw.build_hs(spec, prec, engine, options=_per_step(options))
     ref, rsmon, rstmon = oracle_lib.build_ref(spec, prec, sem)
     for k in (chunks or [steps]):
         net.run(k)
@@ -99,7 +105,7 @@ def test_pipelined_near_far_split(hs, oracle_lib, dlo, dhi):
     it (pull only beyond 2W), with the window at the minimum delay."""
     spec = nw.brunel(N=2000, K=200, seed=12, monitors=True, dlo=dlo, dhi=dhi)
     for prec in (64, 32):
-        net, ref = _compare(spec, prec, "fused", 1, None, oracle_lib, options={2: 50}, chunks=[3, 333, 164])
+        net, ref = _compare(spec, prec, "fused", 1, None, oracle_lib, options={2: 50, 9: 1}, chunks=[3, 333, 164])
         assert net.stats()["window"] == int(round(dlo / 1e-4))
 
 
@@ -264,7 +270,7 @@ def test_reference_bundle_prefs_launch_shapes(hs, engine, options):
     vary, and neuron 3 still spikes at step 4, neuron 4 at step 5."""
     import refcases as rc
     spec, steps, expect = rc.bundle_prefs()
-    net, sm, _ = nw.build_hs(spec, 64, engine, options=options)
+    net, sm, _ = nw.build_hs(spec, 64, engine, options=_per_step(options))
     net.run(steps)
     got = rc.spikes_by_step(*net.spikes(sm[0]))
     assert sorted(got) == sorted(expect)
@@ -305,7 +311,8 @@ def test_cuba_singular_time_constants_refused(hs):
     net.close()
 
 
-@pytest.mark.parametrize("engine,options", [("plain", None), ("fused", None), ("fused", {9: 1}), ("fused", {2: 0})])
+@pytest.mark.parametrize("engine,options", [("plain", None), ("plain", {12: 0}), ("fused", None), ("fused", {12: 0}),
+                                            ("fused", {9: 1}), ("fused", {2: 0})])
 def test_prepare_then_run_same_bits(hs, engine, options):
     """hs_net_prepare instantiates the graphs a run launches without advancing
     the network: prepare + run gives the bits of run alone, and the step count
@@ -313,7 +320,7 @@ def test_prepare_then_run_same_bits(hs, engine, options):
     spec = nw.brunel(N=3000, K=100, seed=9, monitors=True)
     out = []
     for prep in (False, True):
-        net, smon, _ = nw.build_hs(spec, 32, engine, options=options)
+        net, smon, _ = nw.build_hs(spec, 32, engine, options=_per_step(options))
         net.run(300)
         if prep:
             net.prepare(517)
@@ -343,7 +350,7 @@ def test_pipelined_single_step_windows(hs, oracle_lib, prec, which):
     assert ref.events > 1000
 
 
-@pytest.mark.parametrize("opts", [{11: 1}, {11: 1, 9: 1}])
+@pytest.mark.parametrize("opts", [{11: 1}, {11: 1, 12: 0}, {11: 1, 9: 1, 12: 0}])
 def test_cobahh_fast_math_error_vs_fp64(hs, oracle_lib, opts):
     """The FP32 fast form of the COBA HH update (device exponential, hardware
     reciprocal, FMA contraction; option 11) is not reproducible by the oracle

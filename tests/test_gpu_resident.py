@@ -56,6 +56,54 @@ def test_everyone_fires(hs, oracle_lib, n, delays, prec, engine, sem):
         assert _was_resident(net) and ref.events > 0.4 * n * n
 
 
+def _weighted(n, degree, by, seed=7):
+    """n CUBA neurons, each target with `degree` sources per pathway, a weight of its own per synapse or per source."""
+    rng = np.random.default_rng(seed)
+    spec, paths = nw.cuba(N=n, seed=seed, monitors=False), []
+    for var, scale in ((1, 1.5e-3), (2, -3e-3)):
+        pre = np.concatenate([rng.choice(n, degree, replace=False) for _ in range(n)]).astype(np.int32)
+        post = np.repeat(np.arange(n, dtype=np.int32), degree)
+        w = scale * rng.uniform(0.2, 1.0, pre.size if by == rt.HS_W_SYNAPSE else n)
+        o = rng.permutation(pre.size)
+        paths.append(nw.PathSpec(0, 0, var, pre[o], post[o], delay_steps=rng.choice([1, 2, 30], pre.size).astype(np.int32),
+                                 wmode=by, weights=w))
+    spec.paths, spec.spike_monitors, spec.state_monitors = paths, [0], [(0, 0, 0, n)]
+    return spec
+
+
+@pytest.mark.parametrize("by", [rt.HS_W_SYNAPSE, rt.HS_W_PRE])
+@pytest.mark.parametrize("engine,sem", ENGINES)
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n", [65, 1500, 7001])
+def test_weights_of_one_source_each(hs, oracle_lib, n, prec, engine, sem, by):
+    """Every synapse's own weight reaches its own target: one source per target and variable, so no two additions meet
+    and the bits are the oracle's."""
+    net, ref = _compare(_weighted(n, 1, by), prec, engine, sem, None, oracle_lib, chunks=[50, 301, 150])
+    assert _was_resident(net) and ref.events > n
+
+
+@pytest.mark.parametrize("by", [rt.HS_W_SYNAPSE, rt.HS_W_PRE])
+@pytest.mark.parametrize("engine,sem", ENGINES)
+def test_weights_of_many_sources(hs, oracle_lib, engine, sem, by):
+    """The effects of a step on one target are added in any order: at most `degree` additions of a step differ by
+    degree eps times their sum of degree times the largest weight; over the steps the synaptic currents only decay, and a
+    step adds less than them to v."""
+    n, degree, steps = 2000, 40, 400
+    spec = _weighted(n, degree, by)
+    net, smon, st = nw.build_hs(spec, 64, engine)
+    ref, rsmon, rst = oracle_lib.build_ref(spec, 64, sem)
+    net.run(steps)
+    ref.run(steps)
+    assert _was_resident(net) and ref.events > 1000 and net.stats()["events"] == ref.events
+    for x, y in zip(net.spikes(smon[0]), ref.spikes(rsmon[0])):
+        np.testing.assert_array_equal(x, y)
+    atol = steps * degree * np.finfo(np.float64).eps * degree * 3e-3
+    for var in (1, 2):
+        np.testing.assert_allclose(net.get_state(0, var), ref.get_state(0, var), rtol=0, atol=atol)
+    np.testing.assert_allclose(net.state_monitor(st[0], n), ref.state_monitor(rst[0], n), rtol=0, atol=steps * atol)
+    net.close()
+
+
 @pytest.mark.parametrize("opts", [{}, {9: 1}, {9: 1, 4: 2}])
 @pytest.mark.parametrize("engine,sem", ENGINES)
 @pytest.mark.parametrize("spec", ["brunel", "cuba", "cobahh"])
@@ -89,6 +137,20 @@ def test_layout_waits_for_enough_steps(hs):
         net.run(40)
         seen.append(_was_resident(net))
     assert seen == [False, False, True, True]
+    net.close()
+
+
+@pytest.mark.parametrize("n,steps,resident", [(2000, 1534, False), (2000, 1535, True), (1800, 26, False), (1800, 28, True)])
+def test_first_run_over_many_synapses(hs, n, steps, resident):
+    """Beyond 1e6 synapses the first run has to ask for 1500 steps more than the 10 and one per 50,000 synapses that
+    it takes below."""
+    net = rt.Net(32, "fused", 1e-4, 1)
+    spec = nw.brunel(N=n, K=100, seed=2)
+    net.add_group(spec.groups[0].model, n, spec.groups[0].params)
+    pid = net.connect_fixed(0, 0, 0, 625 if n == 2000 else 500, delay=(5e-4, 5e-3), w=(-1e-4, -1e-4))
+    assert net.pathway_info(pid)["nsyn"] == (1250000 if n == 2000 else 900000)
+    net.run(steps)
+    assert _was_resident(net) == resident
     net.close()
 
 
