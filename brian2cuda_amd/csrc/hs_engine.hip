@@ -506,9 +506,11 @@ __global__ __launch_bounds__(256, 8) void hs_k_window_o8(const DGroup<R> *__rest
 
 /* events still in flight at step E = ctl->base (arrival >= E) of spikes emitted
    before E: every spike (i, u) with u >= E - dmax still owes its bundles of
-   delay >= E - u.  One block; the result goes to ctl->pending. */
+   delay >= E - u; those due before step `until`.  One block; the result goes to
+   ctl->pending. */
 template <typename R>
-__global__ __launch_bounds__(256) void hs_k_pending(const DPath<R> *__restrict__ paths, int np, HsCtl *ctl)
+__global__ __launch_bounds__(256) void hs_k_pending(const DPath<R> *__restrict__ paths, int np, HsCtl *ctl,
+                                                    long long until)
 {
     __shared__ unsigned long long part[4];
     const long long E = ctl->base;
@@ -519,12 +521,13 @@ __global__ __launch_bounds__(256) void hs_k_pending(const DPath<R> *__restrict__
         for (long long u = E - dmax; u < E; ++u) {
             const int slot = (int)hs_mod(u, p.Q);
             const int f = (int)max(0LL, E - u - p.dmin); /* first delay slot arriving at or after E */
+            const int l = (int)max((long long)f, min((long long)p.D, until - u - p.dmin));
             for (int s = 0; s < p.nsub; ++s) {
                 const int cnt = p.hist_cnt[((long long)slot * p.nsub + s) * p.cstride];
                 const int32_t *list = p.hist + (long long)slot * p.nsub * p.subcap + (long long)s * p.subcap;
                 for (int k = threadIdx.x; k < cnt; k += blockDim.x) {
                     const long long base = (long long)list[k] * p.D;
-                    acc += (unsigned long long)(p.bstart[base + p.D] - p.bstart[base + f]);
+                    acc += (unsigned long long)(p.bstart[base + l] - p.bstart[base + f]);
                 }
             }
         }
@@ -811,9 +814,9 @@ hipError_t hs_launch_window(const DGroup<R> *groups, int ng, int total_tiles, co
 }
 
 template <typename R>
-hipError_t hs_launch_pending(const DPath<R> *paths, int np, HsCtl *ctl, hipStream_t s)
+hipError_t hs_launch_pending(const DPath<R> *paths, int np, HsCtl *ctl, long long until, hipStream_t s)
 {
-    hipLaunchKernelGGL(hs_k_pending<R>, dim3(1), dim3(256), 0, s, paths, np, ctl);
+    hipLaunchKernelGGL(hs_k_pending<R>, dim3(1), dim3(256), 0, s, paths, np, ctl, until);
     return hipGetLastError();
 }
 
@@ -835,7 +838,7 @@ hipError_t hs_launch_tick(HsCtl *ctl, long long k, hipStream_t s)
     template hipError_t hs_launch_finalize<R>(const DGroup<R> *, int, int, HsCtl *, int, int, hipStream_t);     \
     template hipError_t hs_launch_window<R>(const DGroup<R> *, int, int, const DPath<R> *, int, HsCtl *, int, int, \
                                             int, int, int, int, int, int, hipStream_t);                           \
-    template hipError_t hs_launch_pending<R>(const DPath<R> *, int, HsCtl *, hipStream_t);
+    template hipError_t hs_launch_pending<R>(const DPath<R> *, int, HsCtl *, long long, hipStream_t);
 HS_INSTANTIATE(double)
 HS_INSTANTIATE(float)
 #endif /* !__HIPCC_RTC__ */

@@ -62,7 +62,8 @@ struct HsCtl {
     unsigned long long pending; /* pipelined windows: events of emitted spikes still in flight at base */
     unsigned long long scatter_bad; /* hs_scatter_add: indices outside the target array */
     unsigned long long stalled; /* resident loop: a block waited in vain for the others' spikes */
-    unsigned long long pad_[11];
+    long long ran;              /* and the steps that its last launch ran */
+    unsigned long long pad_[10];
     unsigned long long ev_slot[HS_EV_SLOTS * HS_EV_STRIDE];  /* synaptic events delivered: sum of ev_slot[k*STRIDE] */
     unsigned long long spk_slot[HS_EV_SLOTS * HS_EV_STRIDE]; /* spikes emitted, spread the same way */
 };
@@ -205,9 +206,9 @@ struct HsResArgs {
     const int32_t *off;      /* segment of (pre, block b): syn[off[pre*nb + b] .. off[pre*nb + b + 1]) */
     const HsResSyn<R> *syn;
     unsigned long long *mail; /* [depth][nb][mwords]: a line per block and window (hs_res_header) */
-    unsigned long long *bits; /* [nhist][nb][waves]: spikes of step t as ballots in row t mod nhist */
     HsCtl *ctl;
-    int n, nb, nown, W, dmax, nslots, nhist, depth, mwords, hwords, lanes_log2, list_cap, cap;
+    int n, nb, nown, W, dmax, nslots, depth, mwords, hwords, lanes_log2, list_cap, cap;
+    int most; /* spikes of a window up to which the loop pays (hs_res_most) */
     int nplanes;
     int plane[HS_MAX_VARS];  /* accumulator plane of variable v, or -1 */
     int o_acc, o_evw, o_list, o_list2, o_cnt, o_big, o_evt, o_stage, lds; /* LDS offsets (hs_res_offsets), total */
@@ -215,7 +216,7 @@ struct HsResArgs {
 
 /* a resident run's totals, in host memory */
 struct HsResInfo {
-    long long base;
+    long long base; /* step that it reached */
     unsigned long long events, spikes, records, stalled;
 };
 
@@ -366,14 +367,15 @@ template <typename R>
 hipError_t hs_launch_window(const DGroup<R> *groups, int ng, int total_tiles, const DPath<R> *paths, int np,
                             HsCtl *ctl, int koff, int w, int W, int ms, int block, int n_upd, int n_far, int n_noise,
                             hipStream_t s);
-/* events in flight at ctl->base into ctl->pending */
+/* events in flight at ctl->base, of them those due before step `until`, into ctl->pending */
 template <typename R>
-hipError_t hs_launch_pending(const DPath<R> *paths, int np, HsCtl *ctl, hipStream_t s);
+hipError_t hs_launch_pending(const DPath<R> *paths, int np, HsCtl *ctl, long long until, hipStream_t s);
 hipError_t hs_launch_tick(HsCtl *ctl, long long k, hipStream_t s);
 /* resident step loop (hs_resident.hip).  offsets: the LDS layout; layout: entries
    per (source, block) segment into cnt (and the segments that have any into
    *nonempty), or (write) the entries themselves;
-   resident: nsteps steps from T0, windows numbered from win0 (ms as above: one
+   resident: nsteps steps from T0, or fewer where the network turns out too busy
+   for the loop (ctl->ran), windows numbered from win0 (ms as above: one
    group of a built-in model with synapses); close: spike lists, step base and
    totals after it; refill: the accumulators of the pipelined windows, for a
    network that goes back to them.  a is the host's copy, da the one in HBM */
@@ -387,7 +389,7 @@ template <typename R>
 hipError_t hs_launch_resident(const HsResArgs<R> &a, const HsResArgs<R> *da, const DGroup<R> *g, int ms, int plain,
                               int block, long long T0, int nsteps, uint32_t win0, hipStream_t s);
 template <typename R>
-hipError_t hs_launch_res_close(const HsResArgs<R> &a, const DGroup<R> *g, int block, long long T0, int nsteps,
+hipError_t hs_launch_res_close(const HsResArgs<R> &a, const DGroup<R> *g, long long T0, int nsteps, uint32_t win0,
                                HsResInfo *info, hipStream_t s);
 template <typename R>
 hipError_t hs_launch_res_refill(const DPath<R> *paths, int np, HsCtl *ctl, int W, hipStream_t s);

@@ -34,6 +34,15 @@
  * A block that waits longer than HS_RES_WAIT gives up and sets ctl->stalled;
  * all others then give up as well, so the launch always ends.
  *
+ * A busy network costs the loop more than the per-step forms: every block looks at
+ * every spike (20 ns a spike of a window, against 50 ps an event there), lines that
+ * the lists do not hold are delivered one after another, and a step whose bucket
+ * overflowed takes the spikes of dmax steps.  So each block keeps the balance of
+ * what its windows held beyond a->most spikes; one whose balance exceeds
+ * HS_RES_SLACK windows says so in its header, and since everybody reads every
+ * header of every window, all blocks end after that window.  The host goes on in
+ * the per-step form (hs_res_run).
+ *
  * Measured, us per step before (the per-step form) -> now:
  *   CUBA 4,000 neurons, one-step delay   FP64 plain 8.3 -> 2.4, FP32 fused 5.1 -> 1.9
  *   COBAHH 4,000, no delay               FP64 plain 11.2 -> 6.0
@@ -52,6 +61,10 @@
 
 #define HS_RES_WAIT 500000000LL /* ticks of the 100 MHz wall clock: 5 s */
 #define HS_RES_FEW 64           /* spikes of a line that its polling thread reads by itself */
+#define HS_RES_LINE 64          /* what a line left to the whole block costs, in listed spikes (1.2 us) */
+#define HS_RES_SLACK 128        /* windows of a->most spikes: 1 to 4 ms */
+#define HS_RES_STOP 1
+#define HS_RES_LAST 2
 
 __device__ __forceinline__ HsResSyn<float> hs_res_ld(const HsResSyn<float> *p)
 {
@@ -89,10 +102,11 @@ __device__ __forceinline__ const T *hs_here(const T *p)
 struct HsResShared {
     int nspk[2]; /* this block's spikes of the window and (being emptied) of the next */
     int n1, n2;  /* spikes to deliver: from header words, from lines with more */
-    int nbig, stop;
+    int nbig;
+    int stop; /* HS_RES_STOP: waited in vain; HS_RES_LAST: a header asked for the end of the launch */
+    int replayed; /* spikes of a walk that came from the lists of the launches before */
     int met; /* arrivals of helper waves (hs_res_meet) */
     int wsum[(HS_RES_MAXT + HS_RES_HELPERS) / HS_WAVE];
-    int pad_[1];
 };
 
 template <typename R>
@@ -253,6 +267,7 @@ __device__ __attribute__((noinline)) unsigned int hs_res_replay(const HsResArgs<
             before += v < wid ? S->wsum[v] : 0;
             all += S->wsum[v];
         }
+        if (WALK && threadIdx.x == 0) S->replayed += all;
         for (int c0 = 0; c0 < all; c0 += cap) { /* uniform */
             for (int k = max(0, c0 - before - ex); k < have; ++k) {
                 const int at = before + ex + k - c0;
@@ -269,7 +284,8 @@ __device__ __attribute__((noinline)) unsigned int hs_res_replay(const HsResArgs<
     return ev;
 }
 
-/* a header word: the window's number mod 4096 | up to four spikes of 13 bits, each
+/* a header word: the window's number mod 2048 | whether the block asks for the end of
+   the launch (first word) | up to four spikes of 13 bits, each
    1 + (step offset << 9 | index in the block), 0: none.  A line starts with one
    header word, or two where blocks fire more per window (models with noise: their
    windows are longer); more spikes than they hold: 0x1fff and the count in the
@@ -277,10 +293,12 @@ __device__ __attribute__((noinline)) unsigned int hs_res_replay(const HsResArgs<
    number.  Header words are written every window, so their short number only has
    to differ from those of the windows that used the line last. */
 #define HS_RES_MANY 0x1fffu
+#define HS_RES_WIN(win) ((win) & 0x7ffu) /* beside bits 53 up; depth is below 2048 */
+#define HS_RES_END (1ull << 52)
 
 __device__ __forceinline__ unsigned long long hs_res_header(uint32_t win, int n, int most, const uint16_t *stage)
 {
-    unsigned long long h = (unsigned long long)(win & 0xfffu) << 52;
+    unsigned long long h = (unsigned long long)HS_RES_WIN(win) << 53;
     if (n > most) return h | (unsigned long long)n << 13 | HS_RES_MANY;
     const unsigned long long four = *(const unsigned long long *)stage; /* one LDS read */
 #pragma unroll
@@ -341,7 +359,7 @@ __device__ __attribute__((noinline)) void hs_res_many(const HsResArgs<R> *__rest
                 missing |= (uint32_t)(h[u] >> 32) != win;
             }
         } while (missing && hs_res_wait(a->ctl, &spin, &t0));
-        if (missing) S->stop = 1;
+        if (missing) atomicOr(&S->stop, HS_RES_STOP);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
             for (int p = 0; p < 2; ++p) {
@@ -369,12 +387,12 @@ __device__ __forceinline__ bool hs_res_poll(const HsResArgs<R> *__restrict__ a, 
 #pragma unroll
             for (int k = 0; k < HW; ++k) {
                 const int q = rank + u * nthr;
-                h[u][k] = q < nb ? hs_mail_ld(lines + (uint32_t)(q * mwords) + k) : (unsigned long long)(win & 0xfffu) << 52;
+                h[u][k] = q < nb ? hs_mail_ld(lines + (uint32_t)(q * mwords) + k) : (unsigned long long)HS_RES_WIN(win) << 53;
             }
 #pragma unroll
         for (int u = 0; u < LPT; ++u)
 #pragma unroll
-            for (int k = 0; k < HW; ++k) missing |= (uint32_t)(h[u][k] >> 52) != (win & 0xfffu);
+            for (int k = 0; k < HW; ++k) missing |= (uint32_t)(h[u][k] >> 53) != HS_RES_WIN(win);
     } while (missing && hs_res_wait(a->ctl, &spin, &t0));
     return !missing;
 }
@@ -386,12 +404,13 @@ __device__ __forceinline__ void hs_res_listed(const HsResArgs<R> *__restrict__ a
 {
     unsigned long long h[LPT][HW];
     if (!hs_res_poll<R, LPT, HW>(a, hs_res_lines(a, win), win, rank, nthr, h)) {
-        L.S->stop = 1;
+        atomicOr(&L.S->stop, HS_RES_STOP);
         return;
     }
 #pragma unroll
     for (int u = 0; u < LPT; ++u) {
-        unsigned long long c = h[u][0] & ((1ull << 52) - 1);
+        unsigned long long c = h[u][0] & (HS_RES_END - 1);
+        if (h[u][0] & HS_RES_END) atomicOr(&L.S->stop, HS_RES_LAST);
         if (c == 0) continue;
         const int q = rank + u * nthr;
         if (((uint32_t)c & 0x1fffu) == HS_RES_MANY) {
@@ -401,7 +420,7 @@ __device__ __forceinline__ void hs_res_listed(const HsResArgs<R> *__restrict__ a
         const uint32_t base = (uint32_t)(q * a->nown);
 #pragma unroll
         for (int k = 0; k < HW; ++k) {
-            if (k) c = h[u][k] & ((1ull << 52) - 1);
+            if (k) c = h[u][k] & (HS_RES_END - 1);
             const int n = (c != 0) + ((c >> 13) != 0) + ((c >> 26) != 0) + ((c >> 39) != 0);
             if (n == 0) continue;
             const int at = atomicAdd(&L.S->n1, n);
@@ -435,12 +454,12 @@ __device__ __attribute__((noinline)) unsigned int hs_res_busy(const HsResArgs<R>
                 long long t0 = 0;
                 int spin = 0;
                 while ((uint32_t)(w >> 32) != win && hs_res_wait(a->ctl, &spin, &t0)) w = hs_mail_ld(ln + a->hwords + sp / 2);
-                if ((uint32_t)(w >> 32) != win) L.S->stop = 1;
+                if ((uint32_t)(w >> 32) != win) atomicOr(&L.S->stop, HS_RES_STOP);
                 const uint32_t x = (uint32_t)(w >> (16 * (sp & 1))) & 0xffffu;
                 L.list[k] = (uint32_t)(o * a->nown) + (x & 511u) | (x >> 9) << 20;
             }
             __syncthreads();
-            if (L.S->stop) return ev;
+            if (L.S->stop & HS_RES_STOP) return ev;
             ev += hs_res_deliver<R, PLAIN, WALK>(a, L, m, 0, tb0, from, end, b, threadIdx.x, blockDim.x);
             __syncthreads();
         }
@@ -449,14 +468,16 @@ __device__ __attribute__((noinline)) unsigned int hs_res_busy(const HsResArgs<R>
 }
 
 /* what the polling threads left: listed spikes and busy lines, by all threads of
-   the block (after a barrier); 0 and no further barrier when there is nothing */
+   the block (after a barrier); 0 and no further barrier when there is nothing.  Adds
+   what it costs, in spikes, to *load */
 template <typename R, bool PLAIN, bool WALK>
 __device__ __forceinline__ unsigned int hs_res_rest(const HsResArgs<R> *__restrict__ a, const HsResLds<R> &L,
-                                                    uint32_t win, int b, int tb0, int from, int end)
+                                                    uint32_t win, int b, int tb0, int from, int end, int *load)
 {
     HsResShared *S = L.S;
     const int nbig = S->nbig, n1 = S->n1, n2 = S->n2;
     if (!(nbig | n1 | n2)) return 0;
+    *load += n1 + n2 + HS_RES_LINE * nbig;
     unsigned int ev = hs_res_deliver<R, PLAIN, WALK>(a, L, n1, n2, tb0, from, end, b, threadIdx.x, blockDim.x);
     __syncthreads();
     if (threadIdx.x == 0) S->n1 = S->n2 = S->nbig = 0; /* appended to again after another barrier */
@@ -466,30 +487,34 @@ __device__ __forceinline__ unsigned int hs_res_rest(const HsResArgs<R> *__restri
 
 /* plain form, a bucket that overflowed: the effects due at step T0 + u from the
    spikes of the last dmax steps themselves; nwin: windows of this launch
-   delivered so far */
+   delivered so far.  Returns to thread 0 what it cost, in spikes */
 template <typename R>
-__device__ __attribute__((noinline)) void hs_res_walk(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ g,
+__device__ __attribute__((noinline)) int hs_res_walk(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ g,
                                                       long long T0, uint32_t win0, int u, int nwin)
 {
     const HsResLds<R> L = hs_res_lds(a);
     const int b = hs_res_owner(blockIdx.x, a->nb), W = a->W;
+    if (threadIdx.x == 0) L.S->replayed = 0;
     if (u < a->dmax) (void)hs_res_replay<R, true, true>(a, g, T0, u, u + 1);
+    int load = threadIdx.x == 0 ? L.S->replayed : 0;
     for (int k = max(0, (u - a->dmax) / W); k < nwin; ++k) {
         if (a->hwords == 1) hs_res_listed<R, 4, 1>(a, L, win0 + (uint32_t)k, threadIdx.x, blockDim.x);
         else hs_res_listed<R, 1, 2>(a, L, win0 + (uint32_t)k, threadIdx.x, blockDim.x);
         __syncthreads();
-        if (L.S->stop) return;
-        (void)hs_res_rest<R, true, true>(a, L, win0 + (uint32_t)k, b, 0, u - k * W, 0);
+        if (L.S->stop & HS_RES_STOP) return load;
+        (void)hs_res_rest<R, true, true>(a, L, win0 + (uint32_t)k, b, 0, u - k * W, 0, &load);
         __syncthreads();
     }
+    return load;
 }
 
 /* plain form: the effects due at step T0 + u (slot: its bucket), one after
-   another onto the target variables po[v] (LDS index of this thread's value, or -1) */
+   another onto the target variables po[v] (LDS index of this thread's value, or -1);
+   *load: what a bucket that overflowed costs */
 template <typename R, int NV>
 __device__ __forceinline__ void hs_res_apply(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ g,
                                              const HsResLds<R> &L, const int *po, R *s, long long T0, uint32_t win0,
-                                             int u, int slot, int nwin)
+                                             int u, int slot, int nwin, int *load)
 {
     const int c = L.cnt[slot]; /* the same for every thread */
     if (c == 0) return;
@@ -504,7 +529,7 @@ __device__ __forceinline__ void hs_res_apply(const HsResArgs<R> *__restrict__ a,
             atomicAdd(&L.acc[(t >> 10) * nown + (t & 1023)], L.evw[e0 + e]);
         }
     } else {
-        hs_res_walk(a, g, T0, win0, u, nwin);
+        *load += hs_res_walk(a, g, T0, win0, u, nwin);
     }
     __syncthreads();
 #pragma unroll
@@ -554,6 +579,11 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
     constexpr int NV = HsNV<MS>::value;
     constexpr bool HELP = hs_res_helper<MS>(), NOISY = HELP;
     constexpr int HW = HELP ? 2 : 1; /* header words (a->hwords) */
+    /* fused form: a's fields are then read once and kept, where the compiler would read
+       them again in every step by scalar loads (100,000 neurons FP32 1.82 us a step and
+       1.97, 64 networks 3.8 and 4.05); the plain form, short of registers, gains by
+       those (CUBA 4,000 FP64 2.07 and 2.21) */
+    if constexpr (!PLAIN) (void)hs_here(a);
     const HsResLds<R> L = hs_res_lds(a);
     HsResShared *const S = L.S;
     const int nb = a->nb, nown = a->nown, W = a->W, nslots = a->nslots;
@@ -587,14 +617,18 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
     }
     __syncthreads();
     unsigned int ev = a->dmax ? hs_res_replay<R, PLAIN, false>(a, g, T0, 0, nsteps) : 0u;
+    /* held: spikes and lines of the window before; load: those, and walks, beyond `most` a
+       window (thread 0's count); ask: the block asks for the end of the launch */
+    int most = a->most, held = 0, load = 0;
+    uint32_t ask = 0;
+    asm volatile("" : "+v"(most)); /* the scalar registers are taken */
 
     const int extras = (g->smon_n ? 1 : 0) | (g->rmon_cnt ? 2 : 0);
-    const int hist0 = nsteps - a->nhist; /* steps from here on leave their ballots behind */
     const int slotlen = a->nplanes * nown;
     unsigned int spikes = 0;
     int slot = (int)hs_mod(T0 - 1, nslots); /* slot of the step before the next one */
-    int nwin = 0;
-    for (int t = 0; t < nsteps; t += W, ++nwin) { /* t: step - T0 */
+    int nwin = 0, t = 0, stop; /* t: step - T0 */
+    do {
         const int w = min(W, nsteps - t);
         const uint32_t win = win0 + (uint32_t)nwin;
         const int tb0 = slot + 1 == nslots ? 0 : slot + 1; /* slot of step t */
@@ -602,7 +636,7 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
 #pragma unroll 1
         for (int j = 0; j < w; ++j) {
             if constexpr (PLAIN) {
-                hs_res_apply<R, NV>(a, g, L, po, s, T0, win0, t + j - 1, slot, nwin);
+                hs_res_apply<R, NV>(a, g, L, po, s, T0, win0, t + j - 1, slot, nwin, &load);
             } else {
                 R eff[NV];
                 R *const row = L.acc + slot * slotlen;
@@ -624,7 +658,7 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
             }
             if (valid && hs_step_one<R, MS, !PLAIN>(*g, c, s, k, last, T0 + t + j, i, T0, xj)) bits |= 1u << j;
         }
-        /* the block's spikes of the window: published first, history and monitors after that */
+        /* the block's spikes of the window: published first, monitors after that */
         if (__ballot(bits != 0))
             for (int j = 0; j < w; ++j) {
                 const bool spk = (bits >> j) & 1u;
@@ -642,7 +676,7 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
         unsigned long long *const lines = hs_res_lines(a, win);
         if (tid == 0) {
             unsigned long long *const ln = lines + (uint32_t)(b * a->mwords);
-            hs_mail_st(ln, hs_res_header(win, nspk, 4 * HW, L.stage));
+            hs_mail_st(ln, hs_res_header(win, nspk, 4 * HW, L.stage) | (unsigned long long)ask << 32);
             if (HW == 2) hs_mail_st(ln + 1, hs_res_header(win, nspk > 4 && nspk <= 8 ? nspk - 4 : 0, 8, L.stage + 4));
             S->nspk[(nwin & 1) ^ 1] = 0; /* read by all before the last barrier, counted in after the next */
             spikes += (unsigned int)nspk;
@@ -653,15 +687,9 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
                            (unsigned long long)win << 32 | L.stage[2 * q] |
                                (2 * q + 1 < nspk ? (uint32_t)L.stage[2 * q + 1] << 16 : 0u));
         if (HELP && wid == 0) __builtin_amdgcn_s_setprio(0);
+        load = max(0, load + held - most);
+        ask = load > HS_RES_SLACK * most ? (uint32_t)(HS_RES_END >> 32) : 0u;
         if (!helper) {
-            if (t + w > hist0) {
-                const HsResArgs<R> *h = hs_here(a);
-                for (int j = 0; j < w; ++j) {
-                    const unsigned long long m = __ballot((bits >> j) & 1u);
-                    if (t + j >= hist0 && hs_lane() == 0)
-                        hs_st(h->bits + ((size_t)hs_mod(T0 + t + j, h->nhist) * nb + b) * nwv + wid, m);
-                }
-            }
             if (extras) {
                 const DGroup<R> *h = hs_here(g);
                 if (extras & 2)
@@ -698,8 +726,10 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
                                                          HS_RES_HELPERS);
             }
             __syncthreads();
-            if (S->stop) return; /* uniform: set before a barrier */
+            stop = S->stop; /* uniform: set before a barrier, and the headers are the same for everybody */
+            if (stop & HS_RES_STOP) return;
             const int nbig = S->nbig;
+            held = S->n1 + S->n2 + HS_RES_LINE * nbig; /* (thread 0 reads them before it clears them) */
             if (tid == 0) S->n1 = S->n2 = 0; /* read by all helpers before the barrier, appended to after another */
             if (nbig) { /* lines that hold more than HS_RES_FEW */
                 __syncthreads();
@@ -710,20 +740,24 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
             if ((int)blockDim.x >= nb) hs_res_listed<R, 1, HW>(a, L, win, tid, blockDim.x);
             else hs_res_listed<R, 4, HW>(a, L, win, tid, blockDim.x);
             __syncthreads();
-            if (S->stop) return;
-            ev += hs_res_rest<R, PLAIN, false>(a, L, win, b, tb0, 0, nsteps - t);
+            stop = S->stop;
+            if (stop & HS_RES_STOP) return;
+            held = 0;
+            ev += hs_res_rest<R, PLAIN, false>(a, L, win, b, tb0, 0, nsteps - t, &held);
         }
-        if (S->stop) return;
-    }
+        if (S->stop & HS_RES_STOP) return;
+        t += w;
+        ++nwin;
+    } while (!stop && t < nsteps);
     /* the state after the last step: its effects, then the resets of its spikers */
     if constexpr (PLAIN) {
-        hs_res_apply<R, NV>(a, g, L, po, s, T0, win0, nsteps - 1, slot, nwin);
+        hs_res_apply<R, NV>(a, g, L, po, s, T0, win0, t - 1, slot, nwin, &load);
     } else {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
             if (po[v] >= 0) s[v] = s[v] + L.acc[slot * slotlen + po[v]];
     }
-    const long long Tend = T0 + nsteps;
+    const long long Tend = T0 + t;
     if (valid) {
         if (c.has_reset && (long long)last == Tend - 1) {
 #ifdef HS_CG_MODELS
@@ -740,6 +774,7 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
     }
     const unsigned long long evs = hs_wave_sum((unsigned long long)ev);
     hs_flush_events(evs, a->ctl, (long long)b * (blockDim.x / HS_WAVE) + wid);
+    if (b == 0 && tid == 0) a->ctl->ran = t;
     if (tid == 0 && spikes)
         hs_atomic_add(&a->ctl->spk_slot[(b % HS_EV_SLOTS) * HS_EV_STRIDE], (unsigned long long)spikes);
 }

@@ -67,30 +67,36 @@ __global__ __launch_bounds__(HS_RES_LW *HS_WAVE) void hs_k_res_layout(const DPat
 }
 
 /*
- * After the loop: the spike lists of the last dmax steps (what the next launch
- * replays, and the per-step forms read) from the ballots, one step per block; the
- * last block empties the other ring slots, advances the step base and writes the
+ * After the loop: the spike lists of its last dmax steps (what the next launch
+ * replays, and the per-step forms read) from the blocks' lines, one step per block;
+ * the last block empties the other ring slots, advances the step base and writes the
  * run's totals to host memory.
  */
 template <typename R>
-__global__ __launch_bounds__(256) void hs_k_res_close(const HsResArgs<R> a, const DGroup<R> *__restrict__ gp, int waves,
-                                                      int rows, long long Tend, HsResInfo *info)
+__global__ __launch_bounds__(256) void hs_k_res_close(const HsResArgs<R> a, const DGroup<R> *__restrict__ gp, int rows,
+                                                      long long T0, uint32_t win0, HsResInfo *info)
 {
     const DGroup<R> &g = *gp;
-    const long long rowlen = (long long)g.nsub * g.subcap;
+    const long long rowlen = (long long)g.nsub * g.subcap, Tend = T0 + a.ctl->ran;
     if ((int)blockIdx.x < rows) {
         __shared__ int cnt[32];
         const long long t = Tend - 1 - blockIdx.x;
+        if (t < T0) return; /* the launch ran fewer steps than planned: a list of before */
         const int slot = (int)hs_mod(t, g.Q);
         if (threadIdx.x < 32) cnt[threadIdx.x] = 0;
         __syncthreads();
-        const unsigned long long *words = a.bits + (size_t)hs_mod(t, a.nhist) * a.nb * waves;
-        for (int q = threadIdx.x; q < a.nb * waves; q += blockDim.x) {
-            unsigned long long m = hs_ld(words + q);
-            const int i0 = (q / waves) * a.nown + (q % waves) * HS_WAVE;
-            while (m) {
-                const int i = i0 + __ffsll(m) - 1;
-                m &= m - 1;
+        const uint32_t win = win0 + (uint32_t)((t - T0) / a.W);
+        const unsigned int j = (unsigned int)((t - T0) % a.W); /* step of the window */
+        for (int q = threadIdx.x; q < a.nb; q += blockDim.x) {
+            const unsigned long long *const ln = hs_res_lines(&a, win) + (size_t)q * a.mwords;
+            const unsigned long long h = hs_ld(ln);
+            const bool many = (h & 0x1fffu) == HS_RES_MANY;
+            const int n = many ? (int)(h >> 13) & 0x1fff : 4 * a.hwords;
+            for (int k = 0; k < n; ++k) {
+                const uint32_t x = many ? (uint32_t)(hs_ld(ln + a.hwords + k / 2) >> (16 * (k & 1))) & 0xffffu
+                                        : ((uint32_t)(hs_ld(ln + k / 4) >> (13 * (k & 3))) & 0x1fffu) - 1u;
+                if ((x >> 9) != j) continue; /* (or no spike) */
+                const int i = q * a.nown + (int)(x & 511u);
                 const int sub = (i >> 8) & (g.nsub - 1);
                 const int at = atomicAdd(&cnt[sub], 1);
                 hs_st(g.hist + slot * rowlen + (long long)sub * g.subcap + at, (int32_t)i);
@@ -219,12 +225,11 @@ hipError_t hs_launch_resident(const HsResArgs<R> &a, const HsResArgs<R> *da, con
 }
 
 template <typename R>
-hipError_t hs_launch_res_close(const HsResArgs<R> &a, const DGroup<R> *g, int block, long long T0, int nsteps,
+hipError_t hs_launch_res_close(const HsResArgs<R> &a, const DGroup<R> *g, long long T0, int nsteps, uint32_t win0,
                                HsResInfo *info, hipStream_t s)
 {
     const int rows = a.dmax < nsteps ? a.dmax : nsteps;
-    hipLaunchKernelGGL(hs_k_res_close<R>, dim3(rows + 1), dim3(256), 0, s, a, g, block / HS_WAVE, rows, T0 + nsteps,
-                       info);
+    hipLaunchKernelGGL(hs_k_res_close<R>, dim3(rows + 1), dim3(256), 0, s, a, g, rows, T0, win0, info);
     return hipGetLastError();
 }
 
@@ -241,7 +246,7 @@ hipError_t hs_launch_res_refill(const DPath<R> *paths, int np, HsCtl *ctl, int W
                                                 unsigned long long *, bool, hipStream_t);                                                       \
     template hipError_t hs_launch_resident<R>(const HsResArgs<R> &, const HsResArgs<R> *, const DGroup<R> *, int, int, \
                                               int, long long, int, uint32_t, hipStream_t);                          \
-    template hipError_t hs_launch_res_close<R>(const HsResArgs<R> &, const DGroup<R> *, int, long long, int,         \
+    template hipError_t hs_launch_res_close<R>(const HsResArgs<R> &, const DGroup<R> *, long long, int, uint32_t,    \
                                                HsResInfo *, hipStream_t);                                           \
     template hipError_t hs_launch_res_refill<R>(const DPath<R> *, int, HsCtl *, int, hipStream_t);
 HS_INSTANTIATE(double)

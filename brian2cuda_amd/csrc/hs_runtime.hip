@@ -498,11 +498,15 @@ struct HsResNet {
     int state = 0;       /* 0 not decided yet, 1 laid out, -1 not for this network */
     bool active = false; /* the last run was resident */
     int64_t asked = 0;   /* steps run in the per-step forms so far */
+    /* spikes and events a step, from the last run of 64 steps or more (below 0: not known) */
+    double spike_rate = -1, event_rate = -1;
+    int64_t rate_steps = 0, rate_spikes = 0, rate_events = 0; /* not yet in them */
+    int64_t until = 0, wait = 0; /* too busy for the loop: not before this step; steps it then stayed out */
     int block = 0;
     uint32_t win = 1;    /* number of the next window */
     size_t mail_bytes = 0;
     HsResInfo *info = nullptr; /* pinned */
-    uint64_t ev_bias = 0;      /* events the pipelined windows counted at emission, delivered (and counted) again here */
+    uint64_t ev_bias = 0;      /* events counted twice: at emission by the pipelined windows, or by a launch cut short */
     HsResArgs<double> a64 = {}; /* geometry and pointers, by precision; and their copy in HBM */
     HsResArgs<float> a32 = {};
     void *dargs = nullptr;
@@ -2402,9 +2406,32 @@ static int hs_check_spike_monitors(hs_net *net, int64_t k, bool *resized)
 #define HS_RES_SYN_PER_STEP 50000
 #define HS_RES_BIG 1000000
 #define HS_RES_FIRST_STEPS 1500
+#define HS_RES_OUT 1000 /* steps that a network too busy for the loop stays out of it, the first time */
 
 /* LDS a block may use: the compute unit's 160 KiB, with a margin */
 #define HS_RES_LDS (156 * 1024)
+
+/*
+ * Spikes of a window of the resident loop up to which it is the faster form.  There
+ * a spike costs 20 ns and an event 24 ps beside the window's own time, and lists
+ * of `list` spikes have to hold them; the per-step forms pay 50 ps an event and
+ * `gain` us more than the loop's window by itself.  Measured, us a step per-step /
+ * resident, neurons firing one by one, Sw spikes a window:
+ *   FP32, pipelined windows (gain 4.5 us; 20,000 neurons, windows of 6 steps)
+ *     50 synapses each  Sw 197  2.05/1.74   340  2.10/2.21   671  2.19/3.39   1770  2.46/21.7
+ *     800               Sw 197  3.31/2.27   340  4.22/3.23   671  6.32/5.43   1770  13.9/27.2
+ *   FP32, two launches per window: gain 7 us
+ *   FP32, a launch per step (gain 9 us; 20,000, windows of 2 steps, lists of 840)
+ *     50                Sw 224  5.53/4.00   590  5.97/6.79;  CUBA, lists of 420: 516  5.46/20.2
+ *   FP64 plain (two launches per step: the lists decide; 20,000, windows of 6 steps)
+ *     50                Sw 340  11.2/2.61   671  11.5/3.86   1770  11.9/23.8
+ */
+static int hs_res_most(const hs_net *net, int list, double degree)
+{
+    if (net->engine == HS_ENGINE_PLAIN) return list * 3 / 4;
+    const double gain = net->window == 1 ? 9.0 : net->mode == 4 ? 4.5 : 7.0, spike = 0.020 - 2.6e-5 * degree;
+    return spike * list / 2 < gain ? list / 2 : (int)(gain / spike);
+}
 
 /* geometry of the resident loop, or false: more than one group, a model the
    loop is not compiled for, pathways of other kinds, more neurons than the
@@ -2446,7 +2473,6 @@ static bool hs_res_geometry(hs_net *net)
     if (r.block > HS_RES_MAXT) return false;
     a.dmax = dmax;
     a.nslots = dmax + 1;
-    a.nhist = std::max(1, dmax);
     a.W = std::min(HS_MAX_WINDOW, dmin + 1);
     a.hwords = hs_res_hwords(g.model);
     a.mwords = ((a.hwords + (a.nown * a.W + 1) / 2) + 15) / 16 * 16;
@@ -2454,9 +2480,9 @@ static bool hs_res_geometry(hs_net *net)
     a.lanes_log2 = 0; /* with the layout */
     a.cap = 0;
     const int plain = net->engine == HS_ENGINE_PLAIN;
-    /* the windows whose lines are read: the current one, and in the plain form
-       those that an overflowing bucket reads back */
-    a.depth = plain ? (dmax + a.W - 1) / a.W + 3 : 2;
+    /* the windows whose lines are read: the current one, and those of the last dmax
+       steps, for the spike lists that a launch leaves and for overflowing buckets */
+    a.depth = (dmax + a.W - 1) / a.W + 3;
     hs_res_offsets<R>(&a, plain);
     if (a.lds > HS_RES_LDS) return false;
     if (plain) {
@@ -2465,6 +2491,7 @@ static bool hs_res_geometry(hs_net *net)
         if (a.cap < 16) return false;
         hs_res_offsets<R>(&a, plain);
     }
+    a.most = hs_res_most(net, a.list_cap, (double)total / g.n);
     return true;
 }
 
@@ -2483,7 +2510,6 @@ static int hs_res_layout(hs_net *net)
     int32_t *cnt = nullptr;
     long long *bsum = nullptr;
     r.mail_bytes = sizeof(unsigned long long) * (size_t)a.depth * a.nb * a.mwords;
-    const size_t bits_bytes = sizeof(unsigned long long) * (size_t)a.nhist * a.nb * (r.block / HS_WAVE);
     bool ok = hipMalloc((void **)&cnt, sizeof(int32_t) * (size_t)segs) == hipSuccess &&
               hipMalloc((void **)&bsum, sizeof(long long) * (size_t)(nblk + 1)) == hipSuccess &&
               hipHostMalloc((void **)&r.info, sizeof(HsResInfo), hipHostMallocDefault) == hipSuccess;
@@ -2492,7 +2518,6 @@ static int hs_res_layout(hs_net *net)
     ok = ok && hs_dalloc(net, sizeof(int32_t) * (size_t)(segs + 1), &off, false) == HS_OK &&
          hs_dalloc(net, sizeof(HsResSyn<R>) * (size_t)std::max<int64_t>(total, 1), &syn, false) == HS_OK &&
          hs_dalloc(net, r.mail_bytes, (void **)&a.mail, true) == HS_OK &&
-         hs_dalloc(net, bits_bytes, (void **)&a.bits, false) == HS_OK &&
          hs_dalloc(net, sizeof(HsResArgs<R>), &r.dargs, false) == HS_OK;
     a.off = (const int32_t *)off;
     a.syn = (const HsResSyn<R> *)syn;
@@ -2518,7 +2543,7 @@ static int hs_res_layout(hs_net *net)
     if (cnt) (void)hipFree(cnt);
     if (bsum) (void)hipFree(bsum);
     if (!ok) {
-        void *held[] = {off, syn, a.mail, a.bits, r.dargs};
+        void *held[] = {off, syn, a.mail, r.dargs};
         for (void *p : held) hs_dfree(net, p);
         if (r.info) (void)hipHostFree(r.info);
         r.dargs = nullptr;
@@ -2530,6 +2555,28 @@ static int hs_res_layout(hs_net *net)
     HS_HIP(es);
     r.state = 1;
     return HS_OK;
+}
+
+/* whether a network is too busy for the loop: its windows hold more spikes than pay
+   (a sixth more, once it is in the loop), or the plain form's buckets would be half
+   full (in the loop they show by themselves) */
+template <typename R>
+static bool hs_res_busy(const HsResNet &r, const HsResArgs<R> &a)
+{
+    if (r.active) return r.spike_rate * a.W * 6 > a.most * 7;
+    return r.spike_rate * a.W > a.most || (a.cap > 0 && r.event_rate / a.nb > a.cap / 2);
+}
+
+/* what `steps` steps say about the network's activity */
+static void hs_res_rates(HsResNet &r, int64_t steps, int64_t spikes, int64_t events)
+{
+    r.rate_steps += steps;
+    r.rate_spikes += spikes;
+    r.rate_events += events;
+    if (r.rate_steps < 64) return;
+    r.spike_rate = (double)r.rate_spikes / r.rate_steps;
+    r.event_rate = (double)r.rate_events / r.rate_steps;
+    r.rate_steps = r.rate_spikes = r.rate_events = 0;
 }
 
 /* whether this run of nsteps steps is resident; lays the synapses out on the
@@ -2544,6 +2591,7 @@ static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use)
        and only the per-step forms record them */
     for (const HMon &M : net->m)
         if (M.kind == 3) return HS_OK;
+    if (net->step < r.until) return HS_OK;
     if (r.state == 0) {
         if (!hs_res_geometry<R>(net)) {
             r.state = -1;
@@ -2562,11 +2610,11 @@ static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use)
            14.1 resident; 50,000, 1.5e7, 380 steps 5.4 and 7.1; 20,000, 1.2e7, 300 steps
            3.8 and 4.5); a network that is run again goes on */
         if (total > HS_RES_BIG && r.asked == 0) worth += HS_RES_FIRST_STEPS;
-        if (r.asked + nsteps < worth) return HS_OK;
+        if (r.asked + nsteps < worth || hs_res_busy(r, hs_res_args<R>(r))) return HS_OK;
         HS_TRY(hs_res_layout<R>(net));
         if (r.state < 0) return HS_OK;
     }
-    *use = true;
+    *use = !hs_res_busy(r, hs_res_args<R>(r));
     return HS_OK;
 }
 
@@ -2575,13 +2623,17 @@ static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use)
     return net->prec == HS_F64 ? hs_res_ready<double>(net, nsteps, use) : hs_res_ready<float>(net, nsteps, use);
 }
 
-/* events still in flight at the network's step (ctl->pending) */
-static int hs_pending(hs_net *net, uint64_t *out)
+#define HS_ANY_STEP (1LL << 62)
+
+/* events still in flight at the network's step, of them those due before step `until` (ctl->pending) */
+static int hs_pending(hs_net *net, int64_t until, uint64_t *out)
 {
     if (net->prec == HS_F64)
-        HS_HIP(hs_launch_pending<double>((const DPath<double> *)net->dpaths, (int)net->p.size(), net->ctl, g_rt.stream));
+        HS_HIP(hs_launch_pending<double>((const DPath<double> *)net->dpaths, (int)net->p.size(), net->ctl, until,
+                                         g_rt.stream));
     else
-        HS_HIP(hs_launch_pending<float>((const DPath<float> *)net->dpaths, (int)net->p.size(), net->ctl, g_rt.stream));
+        HS_HIP(hs_launch_pending<float>((const DPath<float> *)net->dpaths, (int)net->p.size(), net->ctl, until,
+                                        g_rt.stream));
     unsigned long long p = 0;
     HS_HIP(hipMemcpyAsync(&p, &net->ctl->pending, sizeof(p), hipMemcpyDeviceToHost, g_rt.stream));
     HS_HIP(hipStreamSynchronize(g_rt.stream));
@@ -2598,7 +2650,7 @@ static int hs_res_enter(hs_net *net)
     if (r.active) return HS_OK;
     if (net->mode == 4 && net->step > 0) {
         uint64_t p = 0;
-        HS_TRY(hs_pending(net, &p));
+        HS_TRY(hs_pending(net, HS_ANY_STEP, &p));
         r.ev_bias += p;
     }
     r.active = true;
@@ -2622,7 +2674,7 @@ static int hs_res_leave(hs_net *net)
             HS_HIP(hs_launch_res_refill<float>((const DPath<float> *)net->dpaths, (int)net->p.size(), net->ctl,
                                                net->window, g_rt.stream));
         uint64_t p = 0;
-        HS_TRY(hs_pending(net, &p));
+        HS_TRY(hs_pending(net, HS_ANY_STEP, &p));
         r.ev_bias -= p;
     }
     r.active = false;
@@ -2682,27 +2734,43 @@ static int hs_res_run(hs_net *net, int64_t nsteps, std::chrono::steady_clock::ti
             *left = end - net->step;
             return HS_OK;
         }
-        HS_HIP(hs_launch_res_close<R>(a, (const DGroup<R> *)net->dgroups, r.block, net->step, (int)k, r.info,
+        HS_HIP(hs_launch_res_close<R>(a, (const DGroup<R> *)net->dgroups, net->step, (int)k, r.win, r.info,
                                       g_rt.stream));
-        r.win += (uint32_t)wins;
-        net->step += k;
-        if (net->step >= end) HS_HIP(hipEventRecord(net->ev1, g_rt.stream));
+        if (net->step + k >= end) HS_HIP(hipEventRecord(net->ev1, g_rt.stream));
         HS_HIP(hipStreamSynchronize(g_rt.stream));
         known = true;
-        if (r.info->stalled || r.info->base != net->step) {
+        const int64_t ran = r.info->base - net->step;
+        if (r.info->stalled || ran < 1 || ran > k) {
             r.state = -2;
-            return hs_fail(HS_ERR_HIP, "resident step loop: a block waited in vain for the others (step %lld of %lld)",
-                           r.info->base, (long long)net->step);
+            return hs_fail(HS_ERR_HIP, "resident step loop: a block waited in vain for the others (step %lld to %lld)",
+                           (long long)net->step, (long long)(net->step + k));
         }
+        r.win += (uint32_t)((ran + a.W - 1) / a.W);
+        net->step += ran;
+        if (ran < k) {
+            /* too busy: the per-step forms go on, for longer each time.  The launch counted
+               the events due in the steps that it did not come to */
+            uint64_t p = 0;
+            HS_TRY(hs_pending(net, net->step - ran + k, &p));
+            r.ev_bias += p;
+            r.wait = std::min<int64_t>(std::max<int64_t>(2 * r.wait, HS_RES_OUT), 1 << 20);
+            r.until = net->step + r.wait;
+            break;
+        }
+        if (k >= r.wait) r.wait = 0;
     }
+    hs_res_rates(r, nsteps - (end - net->step), (int64_t)(r.info->spikes - net->spikes),
+                 (int64_t)(r.info->events - r.ev_bias - net->events));
+    net->events = r.info->events - r.ev_bias;
+    net->spikes = r.info->spikes;
+    *left = end - net->step;
+    if (*left > 0) return HS_OK;
     auto t1 = std::chrono::steady_clock::now();
     float ms_gpu = 0;
     HS_HIP(hipEventElapsedTime(&ms_gpu, net->ev0, net->ev1));
     net->last_gpu_ms = ms_gpu;
     net->last_wall = std::chrono::duration<double>(t1 - t0).count();
     net->last_steps = nsteps;
-    net->events = r.info->events - r.ev_bias;
-    net->spikes = r.info->spikes;
     if (M && (int64_t)r.info->records > M->cap)
         return hs_fail(HS_ERR_OVERFLOW, "spike monitor overflow: %llu records for capacity %lld", r.info->records,
                        (long long)M->cap);
@@ -2767,10 +2835,10 @@ extern "C" int hs_net_run(hs_net *net, int64_t nsteps)
         /* pipelined windows count events at emission: subtract those still in flight */
         if (net->prec == HS_F64)
             HS_HIP(hs_launch_pending<double>((const DPath<double> *)net->dpaths, (int)net->p.size(), net->ctl,
-                                             g_rt.stream));
+                                             HS_ANY_STEP, g_rt.stream));
         else
             HS_HIP(hs_launch_pending<float>((const DPath<float> *)net->dpaths, (int)net->p.size(), net->ctl,
-                                            g_rt.stream));
+                                            HS_ANY_STEP, g_rt.stream));
     }
     float ms = 0;
     HS_HIP(hipEventElapsedTime(&ms, net->ev0, net->ev1));
@@ -2782,8 +2850,10 @@ extern "C" int hs_net_run(hs_net *net, int64_t nsteps)
     HsCtl &c = cbuf[0];
     HS_HIP(hipMemcpyAsync(&c, net->ctl, sizeof(c), hipMemcpyDeviceToHost, g_rt.stream));
     HS_HIP(hipStreamSynchronize(g_rt.stream));
+    const uint64_t events0 = net->events, spikes0 = net->spikes;
     net->events = hs_ctl_events(c) - (net->mode == 4 ? c.pending : 0ull) - net->res.ev_bias;
     net->spikes = hs_ctl_spikes(c);
+    hs_res_rates(net->res, nsteps, (int64_t)(net->spikes - spikes0), (int64_t)(net->events - events0));
     if (c.base != net->step) return hs_fail(HS_ERR_STATE, "device step %lld != host step %lld", c.base, (long long)net->step);
     for (const HMon &M : net->m) {
         if (M.kind != 0 || M.rec >= 0) continue;

@@ -453,7 +453,8 @@ int hs_net_set_monitor_interval(hs_net *net, int mid, int every);
  * 12 resident step loop (1, the default: a network of one built-in group whose
  * pathways are scattered and whose neurons and delays fit the chip runs many
  * steps per launch, its state in registers and LDS, once it is asked for enough
- * steps to pay for laying its synapses out; the same results, whatever keys 0 to
+ * steps to pay for laying its synapses out and while its neurons do not fire more
+ * than the loop is the faster form for; the same results, whatever keys 0 to
  * 10 say; 0: always the per-step forms that they describe, as with key 7).
  * Key 13 can only be read: 1 if the last run was resident.
  * brian2cuda_amd/autotune.py picks keys 0, 1, 3, 4, 8, 9, 10 by measurement in the

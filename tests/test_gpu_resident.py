@@ -219,3 +219,73 @@ def test_run_time_counts_the_layout(hs):
             wall[prepared] = min(wall.get(prepared, 1.0), s["last_run_wall_s"])
             net.close()
     assert wall[False] > 1.5 * wall[True]
+
+
+def _driven(n, degree, mu, delays, seed=5):
+    """n noise-driven neurons that fire as mu says, whatever reaches them: `degree` synapses each; mu None: CUBA neurons
+    well above their threshold."""
+    if mu is None:
+        spec = _cuba(n, degree / n, [int(round(d * 1e4)) for d in delays], we=1e-9, wi=-1e-9)
+        spec.groups[0].params = [-20e-3, *spec.groups[0].params[1:]]
+        spec.state_monitors, spec.rate_monitors = [(0, 0, 0, 7)], [(0, 0, n)]
+        return spec
+    spec = nw.brunel(N=n, K=degree, seed=seed, J=-1e-9, dlo=delays[0], dhi=delays[1], mu=mu, monitors=True)
+    spec.state_monitors, spec.rate_monitors = [(0, 0, 0, 7)], [(0, 0, n)]
+    return spec
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n,degree,mu,delays,engine,sem", [
+    (1500, 200, 0.2, (1e-3, 2e-2), "plain", 0), (1500, 200, 0.2, (1e-4, 5e-3), "plain", 0), (700, 100, 0.2, (0.0, 2e-2), "plain", 0),
+    (4000, 80, None, (7e-4, 3e-3), "plain", 0), (4000, 80, None, (7e-4, 3e-3), "fused", 1),
+    (3000, 100, 0.2, (5e-4, 5e-3), "fused", 1), (3000, 100, 0.2, (2e-4, 3e-4), "fused", 1)])
+def test_busy_networks_leave_the_loop(hs, oracle_lib, n, degree, mu, delays, engine, sem, prec):
+    """A network that turns out too busy ends its launch early, at the same step in all blocks, and goes on in the per-step
+    form with the oracle's bits: spikes, events, monitors, effects in flight."""
+    spec = _driven(n, degree, mu, delays)
+    for opts in ({}, {9: 1}) if engine == "fused" else ({},):
+        net, smon, st = nw.build_hs(spec, prec, engine, options=opts)
+        ref, rsmon, rst = oracle_lib.build_ref(spec, prec, sem)
+        seen = []
+        for k in (20, 1400, 1, 300):
+            net.run(k)
+            ref.run(k)
+            seen.append(_was_resident(net))
+            assert net.stats()["events"] == ref.events and net.stats()["steps"] == sum((20, 1400, 1, 300)[:len(seen)])
+            assert np.array_equal(net.get_state(0, 0), ref.get_state(0, 0))
+        assert seen == [True, False, False, False], seen
+        for a, b in zip(net.spikes(smon[0]), ref.spikes(rsmon[0])):
+            np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(net.state_monitor(st[0], 7), ref.state_monitor(rst[0], 7))
+        np.testing.assert_allclose(net.rate_monitor(net.rate_mids[0]),
+                                   np.bincount(ref.spikes(rsmon[0])[1], minlength=1721) / (n * spec.dt), rtol=1e-12)
+        net.close()
+
+
+def test_busy_networks_do_not_enter(hs):
+    """The rates of the per-step form keep a network out whose windows hold more than the loop's lists."""
+    for mu, resident in ((0.0215, True), (0.2, False)):
+        net, _, _ = nw.build_hs(_driven(3000, 100, mu, (5e-4, 5e-3)), 32, "fused", options={rt.OPT_RESIDENT: 0})
+        net.run(600)
+        net.set_option(rt.OPT_RESIDENT, 1)
+        net.run(100)
+        assert _was_resident(net) == resident
+        net.close()
+
+
+def test_busy_for_a_while(hs):
+    """A network that left the loop comes back once it is quiet, after 1000 steps at the earliest."""
+    net, _, _ = nw.build_hs(_driven(1500, 300, 0.015, (1e-3, 2e-2)), 64, "plain")
+    ref, _, _ = nw.build_hs(_driven(1500, 300, 0.015, (1e-3, 2e-2)), 64, "plain", options={rt.OPT_RESIDENT: 0})
+    seen = []
+    for x in (net, ref):
+        x.set_state(0, 0, np.full(1500, 25e-3))  # everyone fires at once, and rarely after that
+    for k in (20, 500, 400, 400, 300, 50):
+        for x in (net, ref):
+            x.run(k)
+        seen.append(_was_resident(net))
+        assert net.stats()["events"] == ref.stats()["events"] and net.stats()["spikes"] == ref.stats()["spikes"]
+        np.testing.assert_array_equal(net.get_state(0, 0), ref.get_state(0, 0))
+    assert seen == [True, False, False, False, True, True], seen
+    net.close()
+    ref.close()
