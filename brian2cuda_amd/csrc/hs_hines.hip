@@ -60,6 +60,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <memory>
 #include <vector>
 
 #include "../../include/hs.h"
@@ -83,9 +84,13 @@ template <typename R>
 struct HinesDesc {
     const int32_t *tree_comp, *tree_sec;
     const int32_t *order; /* tree of each workgroup */
-    /* per compartment, in the order of place() */
+    /* per compartment, in the caller's order: the state, which a launch reads and writes
+       once, and where the compartment is in the order of hs_h_place, from its tree's first */
     double *v;
     R *m, *n, *h;
+    const int32_t *place;
+    /* per compartment, in the order of hs_h_place */
+    R *wm, *wn, *wh; /* the gates of a launch, where LDS has no room for them */
     const double2 *band; /* superdiagonal, subdiagonal of its row */
     const double *ab1, *cdt, *iext;
     const int32_t *ends; /* nodes at the two ends of each compartment's section: parent | own << 8 */
@@ -465,15 +470,18 @@ __global__ __launch_bounds__(1024) void hs_k_hines(const HinesDesc<R> d, int nst
             ab1[j] = d.ab1[c0 + j];
             cdt[j] = d.cdt[c0 + j];
             iext[j] = d.iext[c0 + j];
-            C.m[j] = d.m[c0 + j];
-            C.n[j] = d.n[c0 + j];
-            C.h[j] = d.h[c0 + j];
             const_cast<int32_t *>(C.ends)[j] = d.ends[c0 + j];
         }
     } else {
-        C = {d.m + c0, d.n + c0, d.h + c0, d.ab1 + c0, d.cdt + c0, d.iext + c0, d.ends + c0};
+        C = {d.wm + c0, d.wn + c0, d.wh + c0, d.ab1 + c0, d.cdt + c0, d.iext + c0, d.ends + c0};
     }
-    for (int j = tid; j < nc; j += blockDim.x) L.V[j] = d.v[c0 + j];
+    for (int j = tid; j < nc; j += blockDim.x) {
+        const int p = d.place[c0 + j];
+        L.V[p] = d.v[c0 + j];
+        C.m[p] = d.m[c0 + j];
+        C.n[p] = d.n[c0 + j];
+        C.h[p] = d.h[c0 + j];
+    }
     if (tid == 0) L.wild[0] = L.wild[1] = L.next[0] = L.next[1] = *L.met = 0;
     __syncthreads();
 
@@ -577,13 +585,13 @@ __global__ __launch_bounds__(1024) void hs_k_hines(const HinesDesc<R> d, int nst
         }
         __syncthreads(); /* the solution and the gates are written */
     }
+    __syncthreads(); /* the potentials are written */
     for (int j = tid; j < nc; j += blockDim.x) {
-        d.v[c0 + j] = L.V[j];
-        if constexpr (INLDS) {
-            d.m[c0 + j] = C.m[j];
-            d.n[c0 + j] = C.n[j];
-            d.h[c0 + j] = C.h[j];
-        }
+        const int p = d.place[c0 + j];
+        d.v[c0 + j] = L.V[p];
+        d.m[c0 + j] = C.m[p];
+        d.n[c0 + j] = C.n[p];
+        d.h[c0 + j] = C.h[p];
     }
     if (spikes) d.spikes[tree] += spikes;
 }
@@ -608,8 +616,8 @@ struct hs_hines {
     HinesDesc<float> d32;
     long long steps_per_launch = 1000;
     int64_t steps = 0;
-    const int32_t *place = nullptr; /* where each compartment's values are */
-    void *stage = nullptr;          /* values of all compartments in the caller's order */
+    std::unique_ptr<int32_t[]> place; /* where each compartment's constants are, from its tree's first */
+    std::vector<int32_t> tree_comp;
     std::vector<double> area, I; /* host copies: the point current is stored as I / area */
     double last_wall = 0, last_gpu_ms = 0;
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -626,15 +634,53 @@ static int hs_h_alloc(hs_hines *H, size_t bytes, void **p)
 }
 
 template <typename T>
-static int hs_h_upload(hs_hines *H, const std::vector<T> &host, const T **dev)
+static int hs_h_upload(hs_hines *H, const T *host, size_t n, const T **dev)
 {
     void *p = nullptr;
-    int r = hs_h_alloc(H, sizeof(T) * host.size(), &p);
+    int r = hs_h_alloc(H, sizeof(T) * n, &p);
     if (r != HS_OK) return r;
-    if (!host.empty())
-        HS_HIP(hipMemcpyAsync(p, host.data(), sizeof(T) * host.size(), hipMemcpyHostToDevice, hs_rt_stream()));
+    if (n) HS_HIP(hipMemcpyAsync(p, host, sizeof(T) * n, hipMemcpyHostToDevice, hs_rt_stream()));
     *dev = (const T *)p;
     return HS_OK;
+}
+
+/* small tables, which go to the device together: an allocation and a copy of their
+   own take 20 us each */
+struct HinesPack {
+    std::vector<char> host;
+    std::vector<std::pair<const void **, size_t>> at;
+};
+
+template <typename T>
+static int hs_h_upload(hs_hines *H, HinesPack &pack, const std::vector<T> &host, const T **dev)
+{
+    const size_t bytes = sizeof(T) * host.size(), o = (pack.host.size() + 255) & ~(size_t)255;
+    if (bytes > 65536) return hs_h_upload(H, host.data(), host.size(), dev);
+    pack.host.resize(o + std::max<size_t>(bytes, 1));
+    if (bytes) memcpy(pack.host.data() + o, host.data(), bytes);
+    pack.at.push_back({(const void **)dev, o});
+    return HS_OK;
+}
+
+static int hs_h_upload(hs_hines *H, const HinesPack &pack)
+{
+    if (pack.at.empty()) return HS_OK;
+    const char *dev = nullptr;
+    const int r = hs_h_upload(H, pack.host.data(), pack.host.size(), &dev);
+    for (const auto &x : pack.at) *x.first = dev + x.second;
+    return r;
+}
+
+/* constants that keep the short divisions away from the ends of the exponent range:
+   zero or of ordinary size */
+static bool hs_h_ordinary(const double *x, size_t n)
+{
+    bool ok = true;
+    for (size_t i = 0; i < n; ++i) {
+        const double m = x[i] < 0 ? -x[i] : x[i];
+        ok &= (m == 0.0) | ((m > 1e-40) & (m < 1e40));
+    }
+    return ok;
 }
 
 /* the pointer and size fields shared by the double and float descriptors */
@@ -646,6 +692,7 @@ static void hs_h_copy_common(HinesDesc<R> &o, const HinesDesc<double> &d)
     o.order = d.order;
     o.row = d.row;
     o.v = d.v;
+    o.place = d.place;
     o.band = d.band;
     o.ab1 = d.ab1;
     o.tree_row = d.tree_row;
@@ -705,50 +752,58 @@ static std::vector<int32_t> hs_h_order(const int32_t *tree_comp, int n, int row)
 static void hs_h_place(int ns, const int32_t *size, int nc, int32_t *place, int32_t *first, int32_t *last, int32_t *len,
                        std::vector<int32_t> *off)
 {
-    std::vector<int> by((size_t)ns), from((size_t)ns);
+    int live[HS_HINES_MAXC + 1], rank[HS_HINES_MAXC + 1]; /* sections with a q-th compartment; the next of a size */
+    const int rows = *std::max_element(size, size + ns);
+    std::fill(live, live + rows, 0);
+    for (int s = 0; s < ns; ++s) ++live[size[s] - 1];
+    for (int q = rows - 2; q >= 0; --q) live[q] += live[q + 1];
+    const size_t o = off->size();
+    off->resize(o + rows + 2 * HS_HINES_PF + 2, nc);
+    int32_t *const row = off->data() + o;
+    row[0] = 0;
+    for (int q = 1; q < rows; ++q) row[q] = row[q - 1] + live[q - 1];
+    for (int z = 1; z <= rows; ++z) rank[z] = z < rows ? live[z] : 0; /* the longer ones come first */
     for (int s = 0, at = 0; s < ns; at += size[s++]) {
-        by[s] = s;
-        from[s] = at;
+        const int r = rank[size[s]]++;
+        len[r] = size[s];
+        for (int q = 0; q < size[s]; ++q) place[at + q] = row[q] + r;
+        first[s] = r;
+        last[s] = row[size[s] - 1] + r;
     }
-    std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return size[a] > size[b]; });
-    int at = 0, live = ns;
-    for (int r = 0; r < ns; ++r) len[r] = size[by[r]];
-    for (int q = 0; q < size[by[0]]; ++q) {
-        while (size[by[live - 1]] <= q) --live;
-        off->push_back(at);
-        for (int r = 0; r < live; ++r) {
-            const int s = by[r];
-            place[from[s] + q] = at + r;
-            if (q == 0) first[s] = at + r;
-            if (q == size[s] - 1) last[s] = at + r;
-        }
-        at += live;
-    }
-    for (int q = 0; q < 2 * HS_HINES_PF + 2; ++q) off->push_back(nc);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void hs_k_hines_place(const int32_t *place, const T *from, T *to, int n, bool back)
+/* a variable of all compartments to the device, and back */
+static int hs_h_put(hs_hines *H, void *var, const void *host, size_t real)
 {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    if (back) to[i] = from[place[i]];
-    else to[place[i]] = from[i];
-}
-
-/* a variable of all compartments between the caller's memory and the device's order */
-template <typename T> static int hs_h_move(hs_hines *H, T *var, T *host, bool back)
-{
-    hipStream_t st = hs_rt_stream();
-    T *stage = (T *)H->stage;
-    const size_t bytes = sizeof(T) * H->ncomp;
-    const dim3 grid((H->ncomp + 255) / 256);
-    if (!back) HS_HIP(hipMemcpyAsync(stage, host, bytes, hipMemcpyHostToDevice, st));
-    hs_k_hines_place<T><<<grid, 256, 0, st>>>(H->place, back ? var : stage, back ? stage : var, H->ncomp, back);
-    HS_HIP(hipGetLastError());
-    if (back) HS_HIP(hipMemcpyAsync(host, stage, bytes, hipMemcpyDeviceToHost, st));
-    HS_HIP(hipStreamSynchronize(st));
+    HS_HIP(hipMemcpyAsync(var, host, real * H->ncomp, hipMemcpyHostToDevice, hs_rt_stream()));
+    HS_HIP(hipStreamSynchronize(hs_rt_stream()));
     return HS_OK;
+}
+
+static int hs_h_take(hs_hines *H, const void *var, void *host, size_t real)
+{
+    HS_HIP(hipMemcpyAsync(host, var, real * H->ncomp, hipMemcpyDeviceToHost, hs_rt_stream()));
+    HS_HIP(hipStreamSynchronize(hs_rt_stream()));
+    return HS_OK;
+}
+
+/* dynamic LDS of a workgroup (HinesLds) */
+static size_t hs_h_lds(int CM, int SM, int RM, size_t real, bool inlds)
+{
+    return sizeof(double) * (5 * (size_t)CM + 3 * (SM + 1)) + sizeof(int) * ((size_t)RM + 6) +
+           (inlds ? 8 + (size_t)CM * (3 * sizeof(double) + 3 * real + sizeof(int32_t)) : 0);
+}
+
+/* waves of a tree: 16 per compute unit over its trees, at least one besides the
+   solvers, at most one besides them per 64 compartments; everything in LDS where all
+   of a compute unit's trees still fit */
+template <typename R> static int hs_h_waves(const HinesDesc<R> &d, int ntrees, bool *inlds)
+{
+    const int solvers = hs_hines_solvers(d.smax), most = solvers + (d.cmax + HS_WAVE - 1) / HS_WAVE;
+    const int trees = (ntrees + hs_rt_cus() - 1) / hs_rt_cus();
+    const int waves = std::min(std::min(most, 16), std::max(solvers + 1, 16 / trees));
+    *inlds = hs_h_lds(d.cmax, d.smax, d.rmax, sizeof(R), true) * std::min(trees, 16 / waves) <= 160 * 1024;
+    return waves;
 }
 
 extern "C" int hs_hines_create(int precision, double dt, int n_trees, const int32_t *tree_comp,
@@ -763,12 +818,15 @@ extern "C" int hs_hines_create(int precision, double dt, int n_trees, const int3
         return hs_rt_fail(HS_ERR_ARG, "hs_hines_create: bad arguments");
     const int NC = tree_comp[n_trees], NS = tree_sec[n_trees];
     /* validate the morphology and derive the tables of the reference's prep */
-    std::vector<double> ab0(NC, 0.0), ab1(NC, 0.0), ab2(NC, 0.0), invr(NC, 0.0);
-    std::vector<double> pab1(NC), pcdt(NC); /* in the order of place() */
-    std::vector<double2> band(NC);
+    double iv[HS_HINES_MAXC], a0[HS_HINES_MAXC], a1[HS_HINES_MAXC], a2[HS_HINES_MAXC]; /* of one tree */
+    /* in the order of hs_h_place */
+    std::unique_ptr<double[]> pab1(new double[NC]), pcdt(new double[NC]);
+    std::unique_ptr<double2[]> band(new double2[NC]);
+    std::unique_ptr<int32_t[]> ends(new int32_t[NC]), place(new int32_t[NC]);
+    bool narrow = dt <= HS_HINES_DTMAX && hs_h_ordinary(chan, 6); /* the short divisions */
     std::vector<double> invr0(NS), invrn(NS), bplus(NS), bminus(NS); /* the last two by rank */
-    std::vector<int32_t> first(NS), endc(NS), mparent(NS), ends(NC, 0);
-    std::vector<int32_t> pfirst(NS), plast(NS), len(NS), place(NC), off, tree_row(1, 0);
+    std::vector<int32_t> first(NS), endc(NS), mparent(NS);
+    std::vector<int32_t> pfirst(NS), plast(NS), len(NS), off, tree_row(1, 0);
     std::vector<int32_t> nchild(NS + n_trees, 0), child((size_t)(NS + n_trees) * HS_HINES_RL, 0);
     std::vector<int32_t> level(NS + n_trees), nlev(n_trees);
     int cmax = 1, smax = 1, rmax = 1;
@@ -804,14 +862,14 @@ extern "C" int hs_hines_create(int precision, double dt, int n_trees, const int3
         for (int k = 0; k <= ns; ++k) maxd = std::max(maxd, depth[k]);
         for (int k = 0; k <= ns; ++k) level[n0 + k] = depth[k];
         nlev[t] = maxd + 1;
-        hs_h_place(ns, sec_n + s0, N, place.data() + c0, pfirst.data() + s0, plast.data() + s0, len.data() + s0, &off);
+        hs_h_place(ns, sec_n + s0, N, place.get() + c0, pfirst.data() + s0, plast.data() + s0, len.data() + s0, &off);
         tree_row.push_back((int32_t)off.size());
         rmax = std::max(rmax, tree_row[t + 1] - tree_row[t]);
         /* spatialstateupdate.cu:39-83, tree-local indices, same operation order */
         const double *ar = area + c0, *r1 = rl1 + c0, *r2 = rl2 + c0, *cm = Cm + c0;
-        double *iv = invr.data() + c0, *a0 = ab0.data() + c0, *a1 = ab1.data() + c0, *a2 = ab2.data() + c0;
         for (int i = 1; i < N; i++) iv[i] = 1.0 / (Ri * (1 / r2[i - 1] + 1 / r1[i]));
-        for (int s = 0; s < ns; s++) iv[first[s0 + s]] = 0;
+        for (int s = 0; s < ns; s++) iv[first[s0 + s]] = 0; /* (the first section's is compartment 0) */
+        a0[0] = a2[N - 1] = 0.0;
         for (int i = 0; i < N; i++) a1[i] = (-(cm[i] / dt) - iv[i] / ar[i]);
         for (int i = 1; i < N; i++) {
             a0[i] = iv[i] / ar[i - 1];
@@ -835,7 +893,8 @@ extern "C" int hs_hines_create(int precision, double dt, int n_trees, const int3
             pab1[p] = a1[i];
             band[p] = make_double2(i < N - 1 ? a0[i + 1] : 0.0, i > 0 ? a2[i - 1] : 0.0);
         }
-        for (int i = 0; i < N; i++) place[c0 + i] += c0;
+        narrow = narrow && hs_h_ordinary(a0, N) && hs_h_ordinary(a1, N) && hs_h_ordinary(a2, N) &&
+                 hs_h_ordinary(pcdt.get() + c0, N);
     }
     hs_hines *H = new hs_hines();
     H->prec = precision;
@@ -849,23 +908,38 @@ extern "C" int hs_hines_create(int precision, double dt, int n_trees, const int3
     HinesDesc<double> d;
     memset(&d, 0, sizeof(d));
     int rr = HS_OK;
+    HinesPack pack;
 #define UP(vec, field)                                    \
-    if (rr == HS_OK) rr = hs_h_upload(H, vec, &d.field);
+    if (rr == HS_OK) rr = hs_h_upload(H, pack, vec, &d.field);
     std::vector<int32_t> tc(tree_comp, tree_comp + n_trees + 1), ts(tree_sec, tree_sec + n_trees + 1);
     const int row = std::max(1, hs_rt_cus());
     std::vector<int32_t> order = hs_h_order(tree_comp, n_trees, row);
     d.row = row;
     UP(order, order)
-    UP(tc, tree_comp) UP(ts, tree_sec) UP(band, band) UP(pab1, ab1) UP(pcdt, cdt) UP(ends, ends)
+#define UPC(arr, field)                                            \
+    if (rr == HS_OK) rr = hs_h_upload(H, arr.get(), (size_t)NC, &d.field);
+    UP(tc, tree_comp) UP(ts, tree_sec) UPC(band, band) UPC(pab1, ab1) UPC(pcdt, cdt) UPC(ends, ends) UPC(place, place)
     UP(tree_row, tree_row) UP(off, off) UP(len, len) UP(pfirst, first) UP(plast, last) UP(mparent, mparent) UP(invr0, invr0) UP(invrn, invrn) UP(bplus, bplus)
     UP(bminus, bminus) UP(nchild, nchild) UP(child, child) UP(level, level) UP(nlev, nlevels)
+#undef UPC
 #undef UP
-    std::vector<double> zeros(NC, 0.0);
-    if (rr == HS_OK) rr = hs_h_upload(H, zeros, &d.iext);
+    if (rr == HS_OK) rr = hs_h_upload(H, pack);
+    d.cmax = cmax;
+    d.smax = smax;
+    d.rmax = rmax;
+    bool inlds;
+    if (precision == HS_F64) {
+        (void)hs_h_waves<double>(d, n_trees, &inlds);
+    } else {
+        hs_h_copy_common(H->d32, d);
+        (void)hs_h_waves<float>(H->d32, n_trees, &inlds);
+    }
+    void *pi = nullptr, *pw[3] = {nullptr, nullptr, nullptr};
     void *pv = nullptr, *pm = nullptr, *pn = nullptr, *ph = nullptr, *ps = nullptr;
     const size_t rs = precision == HS_F64 ? sizeof(double) : sizeof(float);
-    if (rr == HS_OK) rr = hs_h_upload(H, place, &H->place);
-    if (rr == HS_OK) rr = hs_h_alloc(H, sizeof(double) * NC, &H->stage);
+    if (rr == HS_OK) rr = hs_h_alloc(H, sizeof(double) * NC, &pi);
+    for (int q = 0; q < 3; ++q)
+        if (rr == HS_OK && !inlds) rr = hs_h_alloc(H, rs * NC, &pw[q]);
     if (rr == HS_OK) rr = hs_h_alloc(H, sizeof(double) * NC, &pv);
     if (rr == HS_OK) rr = hs_h_alloc(H, rs * NC, &pm);
     if (rr == HS_OK) rr = hs_h_alloc(H, rs * NC, &pn);
@@ -877,6 +951,7 @@ extern "C" int hs_hines_create(int precision, double dt, int n_trees, const int3
     }
     hipStream_t st = hs_rt_stream();
     if (hipMemsetAsync(pv, 0, sizeof(double) * NC, st) != hipSuccess ||
+        hipMemsetAsync(pi, 0, sizeof(double) * NC, st) != hipSuccess ||
         hipMemsetAsync(pm, 0, rs * NC, st) != hipSuccess || hipMemsetAsync(pn, 0, rs * NC, st) != hipSuccess ||
         hipMemsetAsync(ph, 0, rs * NC, st) != hipSuccess ||
         hipMemsetAsync(ps, 0, sizeof(int32_t) * n_trees, st) != hipSuccess ||
@@ -885,25 +960,23 @@ extern "C" int hs_hines_create(int precision, double dt, int n_trees, const int3
         return hs_rt_fail(HS_ERR_HIP, "hs_hines_create: initialising device arrays failed");
     }
     d.v = (double *)pv;
+    d.iext = (const double *)pi;
     d.spikes = (int32_t *)ps;
     d.vth = v_spike;
-    /* the short divisions: every constant of the system zero or of ordinary size, so
-       that no quotient comes near the ends of the exponent range */
-    auto ordinary = [](const std::vector<double> &x) {
-        return std::all_of(x.begin(), x.end(), [](double a) {
-            const double m = a < 0 ? -a : a;
-            return a == 0.0 || (m > 1e-40 && m < 1e40);
-        });
-    };
-    d.narrow = dt <= HS_HINES_DTMAX && ordinary(ab0) && ordinary(ab1) && ordinary(ab2) && ordinary(pcdt) && ordinary(invr0) &&
-               ordinary(invrn) && ordinary(bplus) && ordinary(bminus) && ordinary(std::vector<double>(chan, chan + 6));
-    d.cmax = cmax;
-    d.smax = smax;
-    d.rmax = rmax;
+    d.narrow = narrow && hs_h_ordinary(invr0.data(), NS) && hs_h_ordinary(invrn.data(), NS) &&
+               hs_h_ordinary(bplus.data(), NS) && hs_h_ordinary(bminus.data(), NS);
     H->d64 = d;
     hs_h_copy_common(H->d32, d);
     H->area.assign(area, area + NC);
     H->I.assign(NC, 0.0);
+    H->place = std::move(place);
+    H->tree_comp.assign(tree_comp, tree_comp + n_trees + 1);
+    H->d64.wm = (double *)pw[0];
+    H->d64.wn = (double *)pw[1];
+    H->d64.wh = (double *)pw[2];
+    H->d32.wm = (float *)pw[0];
+    H->d32.wn = (float *)pw[1];
+    H->d32.wh = (float *)pw[2];
     H->d64.m = (double *)pm;
     H->d64.n = (double *)pn;
     H->d64.h = (double *)ph;
@@ -947,18 +1020,19 @@ extern "C" int hs_hines_set_state(hs_hines *H, int var, const double *values)
     if (var == 4) {
         /* a point current enters the membrane equation as the density I / area */
         std::vector<double> ia(H->ncomp);
-        for (int i = 0; i < H->ncomp; ++i) {
-            H->I[i] = values[i];
-            ia[i] = values[i] / H->area[i];
-        }
-        return hs_h_move(H, (double *)p, ia.data(), false);
+        for (int t = 0; t < H->ntrees; ++t)
+            for (int c0 = H->tree_comp[t], i = c0; i < H->tree_comp[t + 1]; ++i) {
+                H->I[i] = values[i];
+                ia[c0 + H->place[i]] = values[i] / H->area[i];
+            }
+        return hs_h_put(H, p, ia.data(), sizeof(double));
     }
     if (gate && H->prec == HS_F32) {
         std::vector<float> f(H->ncomp);
         for (int i = 0; i < H->ncomp; ++i) f[i] = (float)values[i];
-        return hs_h_move(H, (float *)p, f.data(), false);
+        return hs_h_put(H, p, f.data(), sizeof(float));
     }
-    return hs_h_move(H, (double *)p, const_cast<double *>(values), false);
+    return hs_h_put(H, p, values, sizeof(double));
 }
 
 extern "C" int hs_hines_get_state(hs_hines *H, int var, double *values)
@@ -974,11 +1048,11 @@ extern "C" int hs_hines_get_state(hs_hines *H, int var, double *values)
     }
     if (gate && H->prec == HS_F32) {
         std::vector<float> f(H->ncomp);
-        r = hs_h_move(H, (float *)p, f.data(), true);
+        r = hs_h_take(H, p, f.data(), sizeof(float));
         for (int i = 0; i < H->ncomp; ++i) values[i] = f[i];
         return r;
     }
-    return hs_h_move(H, (double *)p, values, true);
+    return hs_h_take(H, p, values, sizeof(double));
 }
 
 extern "C" int hs_hines_set_option(hs_hines *H, int key, long long value)
@@ -988,24 +1062,12 @@ extern "C" int hs_hines_set_option(hs_hines *H, int key, long long value)
     return HS_OK;
 }
 
-/* dynamic LDS of a workgroup (HinesLds) */
-static size_t hs_h_lds(int CM, int SM, int RM, size_t real, bool inlds)
-{
-    return sizeof(double) * (5 * (size_t)CM + 3 * (SM + 1)) + sizeof(int) * ((size_t)RM + 6) +
-           (inlds ? 8 + (size_t)CM * (3 * sizeof(double) + 3 * real + sizeof(int32_t)) : 0);
-}
-
 template <typename R>
-static hipError_t hs_h_launch(const HinesDesc<R> &d, int ntrees, int cmax, int k, hipStream_t s)
+static hipError_t hs_h_launch(const HinesDesc<R> &d, int ntrees, int k, hipStream_t s)
 {
-    /* waves of a tree: 16 per compute unit over its trees, at least one besides the
-       solvers, at most one besides them per 64 compartments */
-    const int solvers = hs_hines_solvers(d.smax), most = solvers + (cmax + HS_WAVE - 1) / HS_WAVE;
-    const int trees = (ntrees + hs_rt_cus() - 1) / hs_rt_cus();
-    const int waves = std::min(std::min(most, 16), std::max(solvers + 1, 16 / trees));
-    /* everything in LDS where all of a compute unit's trees still fit */
-    const bool inlds = hs_h_lds(cmax, d.smax, d.rmax, sizeof(R), true) * std::min(trees, 16 / waves) <= 160 * 1024;
-    const size_t lds = hs_h_lds(cmax, d.smax, d.rmax, sizeof(R), inlds);
+    bool inlds;
+    const int waves = hs_h_waves(d, ntrees, &inlds);
+    const size_t lds = hs_h_lds(d.cmax, d.smax, d.rmax, sizeof(R), inlds);
     const int nn = d.smax + 1; /* nodes per lane of the first solver: 1, 2 or 4 */
     const void *f = inlds ? (nn <= HS_WAVE       ? (const void *)hs_k_hines<R, 1, true>
                              : nn <= 2 * HS_WAVE ? (const void *)hs_k_hines<R, 2, true>
@@ -1033,8 +1095,8 @@ extern "C" int hs_hines_run(hs_hines *H, int64_t nsteps)
     HS_HIP(hipEventRecord(H->e0, st));
     for (int64_t done = 0; done < nsteps;) {
         const int k = (int)std::min<int64_t>(H->steps_per_launch, nsteps - done);
-        if (H->prec == HS_F64) HS_HIP(hs_h_launch<double>(H->d64, H->ntrees, CM, k, st));
-        else HS_HIP(hs_h_launch<float>(H->d32, H->ntrees, CM, k, st));
+        if (H->prec == HS_F64) HS_HIP(hs_h_launch<double>(H->d64, H->ntrees, k, st));
+        else HS_HIP(hs_h_launch<float>(H->d32, H->ntrees, k, st));
         done += k;
     }
     HS_HIP(hipEventRecord(H->e1, st));

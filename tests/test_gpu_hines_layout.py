@@ -71,3 +71,25 @@ def test_outside_the_short_forms(hs, kind, prec):
     if kind == "nan":
         tb.init[1][5] = np.nan
     _check(tb, prec, 40)
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("sizes,n_trees", [([5, 1, 30, 2], 3), ([16] * 40, 520)])
+def test_state_between_launches(hs, sizes, n_trees, prec):
+    """The caller's order of the compartments between launches of a few steps, with the gates of a launch in LDS (3 trees)
+    and in global memory (520 of 640 compartments): states and currents set and read in between."""
+    tb = _combs(sizes, n_trees)
+    g, r = mo.build_hs(tb, prec), oracle.RefMC(tb, prec)
+    g.set_option(0, 3)
+    rng = np.random.default_rng(9)
+    for k in range(2):
+        g.run(7)
+        r.run(7)
+        for var in range(4):
+            np.testing.assert_array_equal(g.get_state(var), r.get_state(var), err_msg=f"var {var}")
+        for var, new in ((0, rng.uniform(-0.02, 0.02, tb.n_comp)), (2, rng.uniform(0, 1, tb.n_comp)),
+                         (4, rng.uniform(0, 1e-11, tb.n_comp))):
+            g.set_state(var, new)
+            r.set_state(var, new)
+            if var != 2:
+                np.testing.assert_array_equal(g.get_state(var), new)
