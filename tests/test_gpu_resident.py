@@ -273,6 +273,25 @@ def test_busy_networks_do_not_enter(hs):
         net.close()
 
 
+@pytest.mark.parametrize("engine,sem", ENGINES)
+def test_short_runs_with_many_spikes_in_flight(hs, oracle_lib, engine, sem):
+    """Single steps of a network whose delays hold 1700 spikes, which the loop's start would deliver again, take the
+    per-step form; longer runs the loop; the bits are the oracle's throughout."""
+    spec = _driven(8000, 50, 0.025, (5e-4, 5e-3))
+    net, smon, _ = nw.build_hs(spec, 64, engine)
+    ref, rsmon, _ = oracle_lib.build_ref(spec, 64, sem)
+    seen = []
+    for k in (300, 1, 1, 50, 1, 120):
+        net.run(k)
+        ref.run(k)
+        seen.append(_was_resident(net))
+        assert net.stats()["events"] == ref.events and np.array_equal(net.get_state(0, 0), ref.get_state(0, 0))
+    assert seen == [True, False, False, True, False, True], seen
+    for a, b in zip(net.spikes(smon[0]), ref.spikes(rsmon[0])):
+        np.testing.assert_array_equal(a, b)
+    net.close()
+
+
 def test_busy_for_a_while(hs):
     """A network that left the loop comes back once it is quiet, after 1000 steps at the earliest."""
     net, _, _ = nw.build_hs(_driven(1500, 300, 0.015, (1e-3, 2e-2)), 64, "plain")
