@@ -159,14 +159,14 @@ template <typename R, int C> struct HsCg;
 template <int MODEL> struct HsNV {
     static constexpr int value = HsCg<double, MODEL - HS_MODEL_CODE>::NV;
 };
-template <int MODEL> __host__ __device__ constexpr bool hs_cg_noisy()
+template <int MODEL> __device__ constexpr bool hs_cg_noisy()
 {
     if constexpr (HS_IS_CODE_MODEL(MODEL)) return HsCg<double, MODEL - HS_MODEL_CODE>::NOISY != 0;
     else return false;
 }
 #else
 template <int MODEL> struct HsNV;
-template <int MODEL> __host__ __device__ constexpr bool hs_cg_noisy() { return false; }
+template <int MODEL> __device__ constexpr bool hs_cg_noisy() { return false; }
 #endif
 template <> struct HsNV<HS_MODEL_LIF_CUBA> { static constexpr int value = HS_LIF_CUBA_NVARS; };
 template <> struct HsNV<HS_MODEL_LIF_NOISE> { static constexpr int value = HS_LIF_NOISE_NVARS; };

@@ -553,7 +553,7 @@ __device__ __forceinline__ void hs_res_meet(HsResShared *S, int arrivals)
    noise (3.6 us for 6 steps of 100,000 FP32 neurons) */
 template <int MS> __host__ __device__ constexpr bool hs_res_helper()
 {
-    return MS == HS_MODEL_LIF_NOISE || hs_cg_noisy<MS>();
+    return MS == HS_MODEL_LIF_NOISE;
 }
 
 /* the n draws of steps T .. T+n-1: independent chains, two at a time, which with
@@ -759,15 +759,7 @@ hs_k_resident(const HsResArgs<R> *__restrict__ a, const DGroup<R> *__restrict__ 
     }
     const long long Tend = T0 + t;
     if (valid) {
-        if (c.has_reset && (long long)last == Tend - 1) {
-#ifdef HS_CG_MODELS
-            if constexpr (HS_IS_CODE_MODEL(MS))
-                HsCg<R, MS - HS_MODEL_CODE>::reset(s, (R)c.dt, (double)(Tend - 1) * c.dt, i, c.seed, c.stream,
-                                                   Tend - 1);
-            else
-#endif
-                s[0] = c.vr;
-        }
+        if (c.has_reset && (long long)last == Tend - 1) s[0] = c.vr;
 #pragma unroll
         for (int v = 0; v < NV; ++v) hs_st(g->var[v] + i, s[v]);
         hs_st(g->last + i, last);
