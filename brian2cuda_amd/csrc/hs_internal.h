@@ -385,6 +385,8 @@ int hs_res_hwords(int ms); /* header words of a line */
 template <typename R>
 hipError_t hs_launch_res_layout(const DPath<R> *paths, int np, const HsResArgs<R> &a, int32_t *cnt,
                                 unsigned long long *nonempty, bool write, hipStream_t s);
+/* the first cooperative launch of a process takes 4 ms (its queue is made): an empty one */
+hipError_t hs_launch_res_first(hipStream_t s);
 template <typename R>
 hipError_t hs_launch_resident(const HsResArgs<R> &a, const HsResArgs<R> *da, const DGroup<R> *g, int ms, int plain,
                               int block, long long T0, int nsteps, uint32_t win0, hipStream_t s);

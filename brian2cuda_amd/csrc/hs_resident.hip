@@ -202,6 +202,14 @@ static hipError_t hs_resident_go(const HsResArgs<R> &a, const HsResArgs<R> *da, 
                                       (unsigned int)a.lds, s);
 }
 
+__global__ void hs_k_res_first() {}
+
+hipError_t hs_launch_res_first(hipStream_t s)
+{
+    void *none[] = {nullptr};
+    return hipLaunchCooperativeKernel((const void *)hs_k_res_first, dim3(1), dim3(HS_WAVE), none, 0, s);
+}
+
 int hs_res_hwords(int ms) { return ms == HS_MODEL_LIF_NOISE ? 2 : 1; }
 
 template <typename R>

@@ -64,6 +64,7 @@ struct HsRuntime {
     int32_t *scratch = nullptr;    /* scratch of the standalone kernels */
     size_t scratch_n = 0;
     double *kbuf = nullptr;        /* constants of hs_stateupdate */
+    bool cooperative = false;      /* a cooperative launch was made (the resident loop) */
 };
 static HsRuntime g_rt;
 
@@ -2510,7 +2511,8 @@ static int hs_res_layout(hs_net *net)
     int32_t *cnt = nullptr;
     long long *bsum = nullptr;
     r.mail_bytes = sizeof(unsigned long long) * (size_t)a.depth * a.nb * a.mwords;
-    bool ok = hipMalloc((void **)&cnt, sizeof(int32_t) * (size_t)segs) == hipSuccess &&
+    if (!g_rt.cooperative) g_rt.cooperative = hs_launch_res_first(g_rt.stream) == hipSuccess;
+    bool ok = g_rt.cooperative && hipMalloc((void **)&cnt, sizeof(int32_t) * (size_t)segs) == hipSuccess &&
               hipMalloc((void **)&bsum, sizeof(long long) * (size_t)(nblk + 1)) == hipSuccess &&
               hipHostMalloc((void **)&r.info, sizeof(HsResInfo), hipHostMallocDefault) == hipSuccess;
     if (!ok) (void)hipGetLastError();
