@@ -31,6 +31,7 @@ of a launch:
   delivery: n_spk*(8 + 12*b) + E*(4 + w_b)   b = delay slots per spike (46),
             w_b = 4 (FP32 per-synapse weight)
   window  : update + delivery (the pipelined form does both in one launch)
+  resident: n_spk*4 + E*(4 + w_b) (the state stays on the chip)
 Bytes and launch time come from one run: when the dominant kernel is the timed
 form's only kernel (the pipelined windows), the timed run itself -- n_spk and E
 its own means, the launch time its HIP events over its launches; otherwise the
@@ -53,7 +54,10 @@ and for the noise-free CUBA and COBAHH networks of 4000 neurons.
 Multicompartment: `--hines-trees` random branched HH trees (100-400
 compartments) advanced `--hines-steps` steps, FP64 and FP32 channel arithmetic;
 its roofline is VALU issue (committed SQ counters per tree-step over the
-measured step time), since the trees stay on chip.
+measured step time, while the kernel's source is the one they were counted on).
+
+The line on stdout holds the headline, both forms, the roofline and a few figures
+of every other part; --report FILE writes all of them, --verbose logs them.
 
 CPU baseline: the oracle (C, cpp_standalone semantics, FP64) on the same
 network -- its OpenMP step loop (bit-identical to the serial one) over
@@ -62,8 +66,10 @@ serial loop on one thread over a bounded window.
 """
 import argparse
 import dataclasses
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -400,13 +406,27 @@ SIMDS, CLOCK_HZ, VALU_CYCLES = 1024, 2.4e9, 4
 VALU_PEAK_GINSTR = SIMDS * CLOCK_HZ / VALU_CYCLES / 1e9
 
 
+def source_tag(*names):
+    """What a profile of a kernel belongs to: a hash of these sources (brian2cuda_amd/csrc) without comments and
+    white space."""
+    h = hashlib.sha256()
+    for name in names:
+        with open(os.path.join(ROOT, "brian2cuda_amd", "csrc", name)) as f:
+            h.update(re.sub(r"\s+", " ", re.sub(r"/\*.*?\*/|//[^\n]*", "", f.read(), flags=re.S)).encode())
+    return h.hexdigest()[:16]
+
+
+HINES_SOURCES = ("hs_hines.hip", "hs_model_body.inc", "hs_detmath.h")
+RESIDENT_SOURCES = ("hs_resident.h",)
+
+
 def hines_valu_roofline(out, prec, n_trees, seed):
-    """hs_k_hines is bound by instruction issue, not by HBM (the trees stay on
-    chip: measured traffic is under 1 B per compartment-step).  achieved = wave
-    VALU instructions issued per second: the committed SQ_INSTS_VALU per
-    tree-step (rocprofv3, profiles/hines_c5_counters.json, the same 2048 trees)
-    x trees / this run's step time; peak = what the SIMDs can issue.  None for
-    another batch.  The HBM figure (68 B per compartment-step, the algorithmic
+    """hs_k_hines is bound by its instructions and their chains, not by HBM.
+    achieved = wave VALU instructions issued per second: the committed
+    SQ_INSTS_VALU per tree-step (rocprofv3, profiles/hines_c5_counters.json, the
+    same 2048 trees) x trees / this run's step time; peak = what the SIMDs can
+    issue.  None for another batch, or once the kernel's source is another one
+    than the counters were taken on.  The HBM figure (68 B per compartment-step, the algorithmic
     byte model) is kept beside it for reference."""
     key = "fp64" if prec == "f64" else "fp32"
     step_s = out[key]["us_per_step"] * 1e-6
@@ -415,13 +435,15 @@ def hines_valu_roofline(out, prec, n_trees, seed):
             "hbm_model_frac": round(hbm / HBM_PEAK_GBS, 6), "bytes_per_compartment_step_model": HINES_BYTES_PER_COMP_STEP,
             "traffic": hines_traffic(n_trees, seed)}
     path = os.path.join(ROOT, "profiles", "hines_c5_counters.json")
-    if n_trees != 2048 or seed != 1234 or not os.path.exists(path):
+    c = None
+    if n_trees == 2048 and seed == 1234 and os.path.exists(path):
+        with open(path) as f:
+            c = json.load(f)
+    if c is None or c["source_tag"] != source_tag(*HINES_SOURCES):
         return {**base, "bound": "valu", "achieved": None, "peak": round(VALU_PEAK_GINSTR, 3),
                 "unit": "G wave-instr/s", "frac": None}
-    with open(path) as f:
-        c = json.load(f)
     k = c["kernels"][f"hs_k_hines_{prec}"]
-    per_tree_step = k["SQ_INSTS_VALU"] / k["SQ_WAVES"] / (c["steps_counted"] / 2)
+    per_tree_step = k["SQ_INSTS_VALU"] / (c["trees"] * c["steps_counted"])
     ach = per_tree_step * n_trees / step_s / 1e9
     return {**base, "bound": "valu", "achieved": round(ach, 3), "peak": round(VALU_PEAK_GINSTR, 3),
             "unit": "G wave-instr/s", "frac": round(ach / VALU_PEAK_GINSTR, 4),
@@ -433,14 +455,16 @@ def hines_valu_roofline(out, prec, n_trees, seed):
 def hines_traffic(n_trees, seed):
     """Measured HBM bytes of one hs_k_hines launch (FP64 and FP32, rocprofv3
     FETCH_SIZE / WRITE_SIZE scaled by a copy of known size) for the batch they
-    were measured on (profiles/hines_c5_traffic.json); None for another batch.
-    A launch reads the trees once and writes them back once, whatever its step
-    count."""
+    were measured on (profiles/hines_c5_traffic.json); None for another batch or
+    another source of the kernel.  The gates of this batch do not fit LDS, so a
+    launch's bytes grow with its steps."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "hines_c5_traffic.json")
     if n_trees != 2048 or seed != 1234 or not os.path.exists(path):
         return None
     with open(path) as f:
         t = json.load(f)
+    if t["source_tag"] != source_tag(*HINES_SOURCES):
+        return None
     out = {}
     for prec in ("f64", "f32"):
         k = t["kernels"][f"hs_k_hines_{prec}"]
@@ -450,8 +474,8 @@ def hines_traffic(n_trees, seed):
     return out
 
 
-def measured_traffic(args, kernel):
-    """HBM bytes per launch of `kernel` from the committed PMC summary
+def measured_traffic(args, kernel, steps):
+    """HBM bytes per launch of `kernel`, of `steps` steps where a launch of it has any number, from the committed PMC summary
     (rocprofv3 --pmc FETCH_SIZE, then WRITE_SIZE, each scaled by what the counter
     reads for a plain copy of known size), for the workload it was measured on;
     None otherwise."""
@@ -461,9 +485,9 @@ def measured_traffic(args, kernel):
     with open(path) as f:
         t = json.load(f)
     k = t["kernels"].get(kernel)
-    if k is None:
+    if k is None or k.get("source_tag", "") not in ("", source_tag(*RESIDENT_SOURCES)):
         return None
-    return int(1024 * (k["fetch_size_kib_per_dispatch"] * t["fetch_scale"] +
+    return int(steps / k.get("steps_per_dispatch", steps) * 1024 * (k["fetch_size_kib_per_dispatch"] * t["fetch_scale"] +
                        k["write_size_kib_per_dispatch"] * t["write_scale"]))
 
 
@@ -597,7 +621,7 @@ def other_configs(args):
             row["fp32_code_model"] = c
             row["code_model_vs_builtin_ms_per_step"] = round(c["ms_per_step"] / f["ms_per_step"], 4)
         out[name] = row
-        log(name, row)
+        log(name, compact_config(row))
     if not args.no_code:
         # C3 with its model as generated code, in the headline's FP32 pipelined form
         cspec = code_spec("brunel_100k", args.seed)
@@ -609,7 +633,7 @@ def other_configs(args):
                                          "fp32_builtin": b,
                                          "code_model_vs_builtin_ms_per_step": round(c["ms_per_step"] /
                                                                                     b["ms_per_step"], 4)}
-        log("brunel_100k_code_model", out["brunel_100k_code_model"])
+        log("brunel_100k_code_model", compact_config(out["brunel_100k_code_model"]))
     return out
 
 
@@ -628,6 +652,43 @@ def code_spec(name, seed):
 def other_spec_brunel(seed):
     from brian2cuda_amd import networks as nw
     return nw.brunel(N=100_000, K=1000, seed=seed)
+
+
+def compact_config(row):
+    """us per step of a configuration's forms and what they are to each other"""
+    us = {k: round(row[k]["ms_per_step"] * 1e3, 3) for k in ("fp32_batched", "fp64_plain", "fp32_fast", "fp32_code_model",
+                                                             "fp32_builtin") if k in row}
+    rel = {k: v for k, v in row.items() if k.startswith(("speedup", "code_model_vs"))}
+    return {"us_per_step": us, **rel,
+            "resident": [k for k in us if row[k].get("resident")]}
+
+
+def compact(out):
+    """the figures that go to stdout: one line that a caller can keep"""
+    form = ("events_per_s", "sim_s_per_wall_s", "ms_per_step", "wall_s", "spikes_per_step", "events_per_step", "window",
+            "resident", "build_s")
+    c = dict(out)
+    for k in ("fp32_batched", "fp64_plain"):
+        if out[k]:
+            c[k] = {f: out[k][f] for f in form}
+    if out["roofline"]:
+        c["roofline"] = {k: v for k, v in out["roofline"].items() if k not in ("kernels", "avg_launch_from")}
+        c["roofline"]["atomics"] = {k: out["roofline"]["atomics"][k] for k in ("achieved_per_s", "scatter_sustained_per_s",
+                                                                               "frac_of_sustained")}
+    if out["other_configs"]:
+        c["other_configs"] = {k: compact_config(r) for k, r in out["other_configs"].items()}
+    dr = c.pop("drift_fp32_batched_vs_fp64_plain")
+    if dr:
+        c["drift"] = {k: {f: r[f] for f in ("rms_dt_steps", "unmatched_frac", "rms_below_1dt_through_steps")}
+                      for k, r in dr.items()}
+    if out["multicompartment"]:
+        m = out["multicompartment"]
+        c["multicompartment"] = {"trees": m["trees"], "compartments": m["compartments"],
+                                 **{f"{p}_us_per_step": m[p]["us_per_step"] for p in ("fp64", "fp32")},
+                                 **{f"{p}_valu_frac": m[f"roofline_{p}"]["frac"] for p in ("fp64", "fp32")}}
+    if out["cpu_baseline"]:
+        c["cpu_baseline"] = {k: v for k, v in out["cpu_baseline"].items() if k != "serial_1_thread"}
+    return c
 
 
 CONFIG_STEPS = 10000  # every configuration simulates 1 s at dt = 0.1 ms
@@ -670,10 +731,13 @@ def main():
     ap.add_argument("--fp64-options", default=None, help="the same for the FP64 plain form")
     ap.add_argument("--no-autotune", action="store_true",
                     help="time both forms with the engine's default launch shapes instead of autotuned ones")
+    ap.add_argument("--report", default=None, help="write every figure of the run to this JSON file")
+    ap.add_argument("--verbose", action="store_true", help="log every figure of the run as it is measured")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only run three 256 MiB device-to-device copies (the reference for scaling the "
                          "FETCH_SIZE / WRITE_SIZE counters of rocprofv3 --pmc) and exit")
     args = ap.parse_args()
+    detail = log if args.verbose else (lambda *a: log(a[0]))
     if args.copy_calibration:
         import torch
         a = torch.ones(64 << 20, dtype=torch.float32, device="cuda")
@@ -717,9 +781,9 @@ def main():
             return nw.build_hs(sp, prec, engine, options=options, device_sort=True)
 
         t0 = time.time()
-        tuned["fp32_batched"] = at.autotune(spec, 32, "fused", build=build, log=log)
+        tuned["fp32_batched"] = at.autotune(spec, 32, "fused", build=build, log=detail if args.verbose else None)
         if not args.no_fp64:
-            tuned["fp64_plain"] = at.autotune(spec, 64, "plain", build=build, log=log)
+            tuned["fp64_plain"] = at.autotune(spec, 64, "plain", build=build, log=detail if args.verbose else None)
         log(f"autotuned in {time.time() - t0:.1f}s: {tuned}")
     fp32 = run_form(spec, 32, "fused", steps, settle, options=tuned["fp32_batched"])
     log("fp32 batched", fp32)
@@ -732,7 +796,7 @@ def main():
     roofline = None
     if args.kt_steps > 0:
         kt, W, kn_spk, kE = kernel_times(spec, 32, "fused", args.kt_steps, settle, options=tuned["fp32_batched"])
-        log("kernel times (fp32 batched)", kt)
+        detail("kernel times (fp32 batched)", kt)
         r_s, w_s = state_bytes(args.workload, 32)
         w_b = weight_bytes(spec, 32)
 
@@ -743,17 +807,17 @@ def main():
                 "hs_k_gather": n_spk * (8 + 12 * D) + E * (4 + w_b),
                 "hs_k_fused": N * (r_s + w_s) + n_spk * (12 + 12 * D) + E * (4 + w_b),
                 "hs_k_window": N * (r_s + w_s) + n_spk * (12 + 12 * D) + E * (4 + w_b),
+                "hs_k_resident": n_spk * 4 + E * (4 + w_b),
             }[name]
 
         name = max(kt, key=lambda k: kt[k]["total_ms"])
         if fp32["resident"]:
             # the timed form's only kernel (the kernel-timed run, an event pair per
-            # launch, takes the per-step kernels instead): the same bytes a step,
-            # over the timed run's own time
+            # launch, takes the per-step kernels instead), over the timed run's own time
             name = "hs_k_resident"
             launches = -(-steps // RESIDENT_STEPS)
             steps_per_launch = steps / launches
-            bpl = per_step("hs_k_window", fp32["spikes_per_step"], fp32["events_per_step"]) * steps_per_launch
+            bpl = per_step(name, fp32["spikes_per_step"], fp32["events_per_step"]) * steps_per_launch
             avg_us = fp32["gpu_ms"] * 1e3 / launches
             src = "timed run: its HIP events over its resident launches; bytes from its own spike and event counts"
             ev_launch = fp32["events_per_step"] * steps_per_launch
@@ -777,7 +841,8 @@ def main():
             ev_launch = kE * steps_per_launch
         achieved = bpl / (avg_us * 1e-6) / 1e9
         roofline = {"bound": "hbm", "achieved": round(achieved, 3), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                    "frac": round(achieved / HBM_PEAK_GBS, 6), "traffic": measured_traffic(args, name),
+                    "frac": round(achieved / HBM_PEAK_GBS, 6),
+                    "traffic": measured_traffic(args, name, steps_per_launch),
                     "kernel": name, "bytes_per_launch": int(bpl), "steps_per_launch": round(steps_per_launch, 3),
                     "avg_launch_us": round(avg_us, 3), "avg_launch_from": src,
                     "avg_launch_us_event_pairs": round(kt[name]["avg_us"], 3) if name in kt else None,
@@ -785,7 +850,7 @@ def main():
         if fp32["resident"]:  # (its effects are LDS atomics: the comparison is per window of the per-step forms)
             ev_launch, avg_us = fp32["events_per_step"] * W, fp32["gpu_ms"] * 1e3 / steps * W
         roofline["atomics"] = atomic_ceiling(N, ev_launch, avg_us, args.seed)
-        log("atomics", roofline["atomics"])
+        detail("atomics", roofline["atomics"])
 
     dr = None
     if args.drift_steps > 0 and not args.no_fp64 and args.workload == "brunel":
@@ -795,7 +860,7 @@ def main():
         # the FP32 fast form of the HH update (option 11): its error against FP64
         dr["cobahh_4k_fp32_fast"] = drift_config(other_spec("cobahh_4k", args.seed), args.drift_steps,
                                                  options={9: 1, 11: 1})
-        log("drift", dr)
+        detail("drift", dr)
 
     others = None
     if args.other_steps > 0 and not args.no_fp64 and args.workload == "brunel":
@@ -806,19 +871,19 @@ def main():
         conn = connect_bench(args)
         conn["host_numpy_generate_s"] = round(spec_s, 4)
         conn["host_bundle_upload_s"] = round(fp32["build_s"], 4)
-        log("connectivity build", conn)
+        detail("connectivity build", conn)
 
     hines = None
     if args.hines_steps > 0:
         hines = hines_bench(args.hines_trees, args.hines_steps, args.seed)
-        log("hines", hines)
+        detail("hines", hines)
 
     cpu = None
     if args.cpu_steps > 0:
         ci = cpu_info()
         threads = args.cpu_threads or min(ci["nproc"], ci["omp_num_threads"] or ci["nproc"])
         cb = cpu_baseline(spec, settle, steps, threads, args.cpu_skip, args.cpu_steps)
-        log("cpu baseline", cb)
+        detail("cpu baseline", cb)
         main_leg = cb.get("threaded", cb["serial"])
         ser = cb["serial"]
         cpu = {"value": round(main_leg["value"], 1), "unit": "synaptic events/s", "cores": main_leg["threads"],
@@ -871,7 +936,10 @@ def main():
         "connectivity_build": conn,
         "device": info,
     }
-    print(json.dumps(out), flush=True)
+    if args.report:
+        with open(args.report, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(compact(out)), flush=True)
 
 
 if __name__ == "__main__":

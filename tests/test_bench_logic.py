@@ -1,4 +1,6 @@
 """Host logic of bench.py (no GPU): the drift matcher and the byte model."""
+import json
+
 import numpy as np
 
 import bench
@@ -51,15 +53,55 @@ def test_drift_horizons_longest_prefix_below_one_step():
     assert "3000" not in rows  # past the run
 
 
-def test_hines_valu_roofline_from_committed_counters():
-    out = {"compartments": 528986, "fp64": {"us_per_step": 31.9}, "fp32": {"us_per_step": 24.0}}
+def test_hines_valu_roofline_from_committed_counters(monkeypatch):
+    out = {"compartments": 528986, "fp64": {"us_per_step": 18.2}, "fp32": {"us_per_step": 13.4}}
     r = bench.hines_valu_roofline(out, "f64", 2048, 1234)
     assert r["bound"] == "valu"
-    # 4,380 wave instructions per tree-step (the committed counters) x 2048 trees / 31.9 us
-    assert abs(r["valu_instr_per_tree_step"] - 4380) < 1
-    assert abs(r["achieved"] - 4380.4 * 2048 / 31.9e-6 / 1e9) < 1
-    assert 0.3 < r["frac"] < 0.6
+    # 3,154 wave instructions per tree-step (the committed counters) x 2048 trees / 18.2 us
+    assert abs(r["valu_instr_per_tree_step"] - 3154) < 1
+    assert abs(r["achieved"] - 3153.8 * 2048 / 18.2e-6 / 1e9) < 1
+    assert 0.4 < r["frac"] < 0.7
     assert bench.hines_valu_roofline(out, "f64", 100, 1234)["frac"] is None  # another batch: no counters
+    assert r["traffic"]["f64_steps_per_launch_measured"] == 200
+    # counters of another kernel than the one in the tree are no measurement of it
+    monkeypatch.setattr(bench, "source_tag", lambda *names: "0" * 16)
+    r = bench.hines_valu_roofline(out, "f64", 2048, 1234)
+    assert r["frac"] is None and r["achieved"] is None and r["traffic"] is None
+
+
+def test_source_tag_ignores_comments_and_space(tmp_path, monkeypatch):
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    d = tmp_path / "brian2cuda_amd" / "csrc"
+    d.mkdir(parents=True)
+    texts = ["int f(int x)\n{\n    return x + 1; /* one\n more */\n}\n", "int f(int x)\n{ return x + 1; // 1\n}\n", "int f(int x) { return x + 2; }"]
+    tags = []
+    for t in texts:
+        (d / "k.hip").write_text(t)
+        tags.append(bench.source_tag("k.hip"))
+    assert tags[0] == tags[1] != tags[2]
+
+
+def test_compact_line_keeps_the_contract_and_fits():
+    form = {k: 0.123456 for k in ("events_per_s", "sim_s_per_wall_s", "ms_per_step", "wall_s", "spikes_per_step",
+                                  "events_per_step", "window", "resident", "build_s", "gpu_ms", "options")}
+    row = {"neurons": 1, "fp32_batched": form, "fp64_plain": form, "fp32_fast": form, "speedup_fp32_batched_vs_fp64_plain": 2.0}
+    drift = {"rms_dt_steps": 1.0, "unmatched_frac": 0.1, "rms_below_1dt_through_steps": 700, "by_horizon": {str(k): row for k in range(20)}}
+    contract = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+                "vs_baseline", "dtype", "data", "config")
+    out = {**{k: "x" * 40 for k in contract}, "fp32_batched": form, "fp64_plain": form,
+           "roofline": {"bound": "hbm", "frac": 0.1, "kernels": {"a": {}}, "avg_launch_from": "x" * 100,
+                        "atomics": {k: 1.0 for k in ("achieved_per_s", "scatter_sustained_per_s", "frac_of_sustained", "x")}},
+           "cpu_baseline": {"value": 1.0, "serial_1_thread": {"a": 1}, "sample": "x" * 300},
+           "other_configs": {f"config_{k}": row for k in range(6)},
+           "drift_fp32_batched_vs_fp64_plain": {f"net_{k}": drift for k in range(4)},
+           "multicompartment": {"trees": 1, "compartments": 2, **{p: {"us_per_step": 1.0} for p in ("fp64", "fp32")},
+                                **{f"roofline_{p}": {"frac": 0.5} for p in ("fp64", "fp32")}}}
+    c = bench.compact(out)
+    assert all(c[k] == out[k] for k in contract)
+    assert len(json.dumps(c)) < 4000
+    assert c["other_configs"]["config_0"]["us_per_step"]["fp64_plain"] == 123.456
+    assert bench.compact({**out, "fp64_plain": None, "roofline": None, "cpu_baseline": None, "other_configs": None,
+                          "drift_fp32_batched_vs_fp64_plain": None, "multicompartment": None})["value"] == out["value"]
 
 
 def test_cpu_info_reports_cores():
