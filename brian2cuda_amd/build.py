@@ -43,7 +43,7 @@ HIPCC_FLAGS = [
 
 # hs_resident.hip, hs_hines.hip: the polynomials' 64-bit constants stay where they are used (two
 # scalar moves) instead of being hoisted out of the step loop, where they exceed
-# the scalar registers and are spilled (254 -> 76 spills in the FP64 noise model)
+# the scalar registers and are spilled (231 -> 52 spills in the FP64 plain noise model)
 SOURCE_FLAGS = {f: ["-mllvm", "-disable-machine-licm"] for f in ("hs_resident.hip", "hs_hines.hip")}
 
 

@@ -43,12 +43,13 @@
  * header of every window, all blocks end after that window.  The host goes on in
  * the per-step form (hs_res_run).
  *
- * Measured, us per step before (the per-step form) -> now:
- *   CUBA 4,000 neurons, one-step delay   FP64 plain 8.3 -> 2.4, FP32 fused 5.1 -> 1.9
- *   COBAHH 4,000, no delay               FP64 plain 11.2 -> 6.0
+ * Measured, us per step of a network that has changed over, readback included; the
+ * per-step form -> the loop:
+ *   CUBA 4,000 neurons, one-step delay   FP64 plain 8.3 -> 2.2, FP32 fused 5.1 -> 1.9
+ *   COBAHH 4,000, no delay               FP64 plain 11.3 -> 6.1
  *   Brunel 20,011, delays 5 to 50        FP64 plain 11.2 -> 2.2
- *   Brunel 100,000, 1e8 synapses         FP32 pipelined 3.67 -> 1.9
- *   64 CUBA networks, 128,000 neurons    FP32 fused 6.9 -> 4.4
+ *   Brunel 100,000, 1e8 synapses         FP32 pipelined 3.68 -> 1.88
+ *   64 CUBA networks, 128,000 neurons    FP32 fused 6.9 -> 4.5
  * What bounds it now is latency: of a CUBA window of 2 steps (3.8 us) the update
  * takes 0.8, the exchange 1.5, segment bounds and entries 1.0; of a 100,000-neuron
  * Brunel window of 6 steps (10.7 us) the noise takes 3.5 and beside it the exchange

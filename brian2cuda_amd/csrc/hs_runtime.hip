@@ -2627,11 +2627,14 @@ static int hs_res_ready(hs_net *net, int64_t nsteps, bool *use)
         int64_t total = 0;
         for (const HPath &P : net->p) total += P.nsyn;
         int64_t worth = HS_RES_MIN_STEPS + total / HS_RES_SYN_PER_STEP;
-        /* beyond HS_RES_BIG synapses the allocations and their release are another 2 ms: a
-           first run has to earn them by itself (a script of one run: 20,000 neurons, 4e6
-           synapses, 100 steps, built and taken down, 12.3 ms in the per-step forms and
-           14.1 resident; 50,000, 1.5e7, 380 steps 5.4 and 7.1; 20,000, 1.2e7, 300 steps
-           3.8 and 4.5); a network that is run again goes on */
+        /* beyond HS_RES_BIG synapses the allocations and their release are another 1 to 3 ms:
+           a first run has to earn them by itself.  1500 steps are what the form that gains
+           least needs, FP32 in pipelined windows (a run and the network's release, per-step
+           form and loop: 100,000 neurons, 1e8 synapses, 1000 steps 4.7 and 6.5 ms, 2000
+           8.2 and 8.0; 50,000, 5e7, 1000 steps 5.9 and 6.6).  The others would earn them
+           sooner (64 CUBA networks, one launch a step, 400 steps 3.5 and 3.6, 1600 10.6
+           and 7.9; 20,000, 5e6, FP64 plain, 100 steps 2.5 and 2.1, 600 8.6 and 3.1): they
+           change over with their second run */
         if (total > HS_RES_BIG && r.asked == 0) worth += HS_RES_FIRST_STEPS;
         if (r.asked + nsteps < worth || hs_res_busy(r, hs_res_args<R>(r))) return HS_OK;
         HS_TRY(hs_res_layout<R>(net));
